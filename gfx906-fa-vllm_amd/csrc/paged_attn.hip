@@ -69,6 +69,11 @@ struct AttnParams {
     const int32_t *bt;
     int64_t bt_stride;
     const int32_t *seq_lens, *qsl, *q_abs;
+    // Padded batches (qsl == nullptr): every sequence has uq query tokens, the
+    // first of sequence s at token row s * uq_rows of q and out (a contiguous
+    // [B, Hq, Sq, 128] tensor with token stride 128 has uq_rows = Hq * Sq).
+    // kv_cap: keys of every sequence without seq_lens, and their bound with.
+    int uq, uq_rows, kv_cap;
     int causal;
     int Hkv, G, block_size;
     float scale_log2e;
@@ -108,6 +113,7 @@ struct AttnParams {
     // the prefill workgroups then copy them into LDS instead of dequantizing
     // every tile themselves.
     uint8_t *pf_tiles;
+    int pf_img_seq;     // > 0: images of every key tile are there, this many per sequence (flat attention)
     int *pf_tbase;      // per sequence (num_seqs + 1): first image tile
     int64_t pf_tiles_cap;
     // Fused cache write of the step's new tokens (decode kernels only; nullptr:
@@ -117,6 +123,13 @@ struct AttnParams {
     int64_t nk_ts, nk_hs, nv_ts, nv_hs;  // element strides
     const int64_t *new_slot;
 };
+
+__device__ __forceinline__ int seq_q0(const AttnParams &p, int s) { return p.qsl ? p.qsl[s] : s * p.uq_rows; }
+__device__ __forceinline__ int seq_nq(const AttnParams &p, int s) { return p.qsl ? p.qsl[s + 1] - p.qsl[s] : p.uq; }
+__device__ __forceinline__ int seq_len(const AttnParams &p, int s) {
+    if (p.kv_cap == INT32_MAX) return p.seq_lens[s];
+    return p.seq_lens ? min(max(p.seq_lens[s], 0), p.kv_cap) : p.kv_cap;
+}
 
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -1339,15 +1352,15 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
         s = blockIdx.y;
         rt = (gridDim.x / Hkv) - 1 - (int)(blockIdx.x / Hkv);
     }
-    const int q0 = p.qsl[s];
-    const int nq = p.qsl[s + 1] - q0;
+    const int q0 = seq_q0(p, s);
+    const int nq = seq_nq(p, s);
     const int nrows = nq * p.G;
     if (nq <= 0 || nrows <= p.dec_rows_max) return;  // uniform over the workgroup
     const int row0 = ROWS * rt;
     if (row0 >= nrows) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int sl = p.seq_lens[s];
+    const int sl = seq_len(p, s);
     const int qa = p.q_abs ? p.q_abs[s] : sl - nq;
     const int jlast = (min(row0 + ROWS, nrows) - 1) / p.G;
     const int kv_end = p.causal ? min(sl, max(qa + jlast + 1, 0)) : sl;
@@ -1367,7 +1380,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
         // fetch until its dequant, one iteration before the consumers read it.
         const int wsp = w - PF_CWAVES;
         // (no images for KS = 2 tiles: the host never passes them there)
-        if (KS == 1 && p.pf_tiles != nullptr && p.pf_count[2] != 0) {  // uniform
+        if (KS == 1 && p.pf_tiles != nullptr && (p.pf_img_seq > 0 || p.pf_count[2] != 0)) {  // uniform
             // The tiles are dequantized images in the workspace.  Copy batch
             // b (K^ of tile b/2 for even b, V^T for odd b) goes from the image
             // straight into its LDS stage in half-step b - 4 and has landed by
@@ -1379,7 +1392,8 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             // batches may still be in flight), or vmcnt(0) near the end, where
             // fewer batches follow.
             const int64_t istride = (int64_t)Hkv * PF_IMG_BYTES;
-            const uint8_t *img0 = p.pf_tiles + ((int64_t)(p.pf_tbase[s] + ktb) * Hkv + h) * PF_IMG_BYTES;
+            const int64_t tb = p.pf_img_seq > 0 ? (int64_t)s * p.pf_img_seq : (int64_t)p.pf_tbase[s];
+            const uint8_t *img0 = p.pf_tiles + ((tb + ktb) * Hkv + h) * PF_IMG_BYTES;
             auto copy = [&](int b) __attribute__((always_inline)) {
                 const int t = b >> 1;
                 if (t >= ntk) return;  // uniform
@@ -1992,8 +2006,8 @@ struct PlSeq {
 
 __device__ __forceinline__ PlSeq pl_seq(const AttnParams &p, int s) {
     PlSeq q;
-    q.nq = p.qsl[s + 1] - p.qsl[s];
-    q.sl = p.seq_lens[s];
+    q.nq = seq_nq(p, s);
+    q.sl = seq_len(p, s);
     q.qa = p.q_abs ? p.q_abs[s] : q.sl - q.nq;
     return q;
 }
@@ -2323,6 +2337,94 @@ __global__ __launch_bounds__(64 * PF_NSP) void prefill_tiles_kernel(AttnParams p
     }
 }
 
+// Tile images of contiguous inputs (the op module's forward()): image
+// (s * nkt + kt) * Hkv + h holds K^ and V^T of keys 64 kt .. 64 kt + 63 of
+// (batch row s, kv-head h), dequantized from the AoS Q8_0 K rows [136 B] and
+// copied from the fp16 V rows [256 B] as they lie in memory; keys past Skv are
+// zeros.  One workgroup per image: its rows are one contiguous run of each
+// input (8704 B and 16384 B), staged through LDS, where a thread picks up one
+// Q8_0 block of one token for K^, and eight tokens of one d for V^T.  The V
+// pitch of 65 dwords spreads a wave's 8 token groups x 8 columns over the
+// banks.  Bound by HBM (25.1 KB read, 35.8 KB written per image) from a few
+// hundred images on, by latency below.  The planar repacking that it took the
+// place of ran one thread per byte of K and per value of V (two launches,
+// 10.8 us at 2048 keys x 4 kv-heads).
+struct FlatTiles {
+    const uint8_t *k;   // [B * Hkv * Skv][136]
+    const uint8_t *v;   // [B * Hkv * Skv][256 B]
+    uint8_t *img;
+    int Hkv, Skv, nkt;
+    int k8, v16;        // bases aligned for 8-byte K and 16-byte V loads
+    float kmul;
+};
+constexpr int FT_VPITCH = 260;
+
+__global__ __launch_bounds__(256) void flat_tiles_kernel(FlatTiles p) {
+    __shared__ __attribute__((aligned(16))) uint8_t sk[PF_TK * 136];
+    __shared__ __attribute__((aligned(16))) uint8_t sv[PF_TK * FT_VPITCH];
+    const int tid = threadIdx.x;
+    const int64_t i = blockIdx.x;
+    const int h = (int)(i % p.Hkv);
+    const int64_t t = i / p.Hkv;
+    const int kt = (int)(t % p.nkt);
+    const int64_t row0 = ((t / p.nkt) * p.Hkv + h) * p.Skv + (int64_t)PF_TK * kt;
+    const int nt = min(p.Skv - PF_TK * kt, PF_TK);  // valid tokens (uniform)
+    const uint8_t *kg = p.k + row0 * 136, *vg = p.v + row0 * 256;
+    const int kb = nt * 136, vb = nt * 256;
+    if (p.v16) {
+#pragma unroll
+        for (int j = 0; j < PF_TK * 256 / (16 * 256); ++j) {
+            const int o = 16 * (tid + 256 * j);
+            const u32x4 x = o < vb ? *reinterpret_cast<const u32x4 *>(vg + o) : u32x4{0, 0, 0, 0};
+            uint32_t *d = reinterpret_cast<uint32_t *>(sv + (o >> 8) * FT_VPITCH + (o & 255));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[e] = x[e];
+        }
+    } else {
+        for (int o = 2 * tid; o < PF_TK * 256; o += 2 * 256)
+            *reinterpret_cast<uint16_t *>(sv + (o >> 8) * FT_VPITCH + (o & 255)) =
+                o < vb ? *reinterpret_cast<const uint16_t *>(vg + o) : (uint16_t)0;
+    }
+    if (p.k8) {
+#pragma unroll
+        for (int j = 0; j < (PF_TK * 136 + 8 * 256 - 1) / (8 * 256); ++j) {
+            const int o = 8 * (tid + 256 * j);
+            if (o < PF_TK * 136)
+                *reinterpret_cast<u32x2 *>(sk + o) = o < kb ? *reinterpret_cast<const u32x2 *>(kg + o) : u32x2{0, 0};
+        }
+    } else {
+        for (int o = tid; o < PF_TK * 136; o += 256) sk[o] = o < kb ? kg[o] : (uint8_t)0;
+    }
+    __syncthreads();
+    uint8_t *img = p.img + i * PF_IMG_BYTES;
+    {   // K^: token tk, Q8_0 block b (32 d); blocks start on 2-byte boundaries
+        const int tk = tid >> 2, b = tid & 3;
+        const uint16_t *blk = reinterpret_cast<const uint16_t *>(sk + tk * 136 + 34 * b);
+        const float sc = half_bits_to_f32(blk[0]) * p.kmul;
+        half8_t *dst = reinterpret_cast<half8_t *>(img + tk * PF_KPITCH + 64 * b);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t w0 = blk[1 + 4 * c] | ((uint32_t)blk[2 + 4 * c] << 16);
+            const uint32_t w1 = blk[3 + 4 * c] | ((uint32_t)blk[4 + 4 * c] << 16);
+            dst[c] = scale8_f32(i8x8_to_half8(w0, w1), sc);
+        }
+    }
+    // V^T: 16-byte chunk c of row d holds positions 8c .. 8c + 7, the tokens
+    // 16 (c / 2) + 4 (c % 2 + 2 (e / 4)) + e % 4 (key bits 2 and 3 swapped)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int c = tid & 7, d = (tid >> 3) + 32 * j;
+        const uint8_t *src = sv + (16 * (c >> 1) + 4 * (c & 1)) * FT_VPITCH + 2 * d;
+        uint16_t x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            x[e] = *reinterpret_cast<const uint16_t *>(src + (8 * (e >> 2) + (e & 3)) * FT_VPITCH);
+        *reinterpret_cast<u32x4 *>(img + PF_KBYTES + d * PF_VPITCH + 16 * c) =
+            u32x4{x[0] | ((uint32_t)x[1] << 16), x[2] | ((uint32_t)x[3] << 16), x[4] | ((uint32_t)x[5] << 16),
+                  x[6] | ((uint32_t)x[7] << 16)};
+    }
+}
+
 // Merges the pieces of each split row tile: per row, an online merge of the
 // pieces' (m, l, O) - the running sums rescaled to the largest m so far - and
 // O divided by l at the end (0 for a row no piece saw a key of).  A unit is 16
@@ -2343,8 +2445,8 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(AttnParams p)
         const int rg = t % (prows / RPU);
         const int *e = p.pf_split + 4 * (t / (prows / RPU));
         const int s = e[0], rt = e[1], slot0 = e[2], k = e[3];
-        const int q0 = p.qsl[s];
-        const int nrows = (p.qsl[s + 1] - q0) * p.G;
+        const int q0 = seq_q0(p, s);
+        const int nrows = seq_nq(p, s) * p.G;
         float M[2], L[2];
         float4_t acc[2];
         int64_t reg0[2];
@@ -2434,9 +2536,10 @@ struct FlatParams {
     int64_t q_ts, q_hs;
     const uint8_t *k;       // AoS Q8_0 rows, [B * Hkv * Skv][136]
     const uint8_t *v;       // fp16 rows, [B * Hkv * Skv][256 B]
-    const int32_t *kv_len;  // [B]: keys each batch row sees (clamped to [0, Skv])
+    const int32_t *kv_len;  // [B]: keys each batch row sees (clamped to [0, Skv]); nullptr: all Skv
     const int32_t *q_abs;   // [B] or nullptr: row j sees keys <= q_abs[b] + j
     int B, Hkv, G, Sq, Skv, P, nsp;
+    int brows;              // token rows of q and out from one batch row to the next
     float c;                // scale * log2 e
     float *out;             // fp32 [B * Sq][Hq][128]
     int64_t o_ts, o_hs;
@@ -2451,7 +2554,7 @@ __global__ __launch_bounds__(64) void flat_decode_kernel(FlatParams p) {
     const int lane = threadIdx.x, i16 = lane & 15, g = lane >> 4;
     const int seg = blockIdx.x / p.P, pc = blockIdx.x - seg * p.P;
     const int b = seg / p.Hkv, h = seg - b * p.Hkv;
-    const int kvl = min(max(p.kv_len[b], 0), p.Skv);
+    const int kvl = p.kv_len ? min(max(p.kv_len[b], 0), p.Skv) : p.Skv;
     const int s0 = (int)((int64_t)pc * p.nsp / p.P);
     const int s1 = min((int)((int64_t)(pc + 1) * p.nsp / p.P), (kvl + 15) >> 4);
     const int n = max(s1 - s0, 0);
@@ -2462,7 +2565,7 @@ __global__ __launch_bounds__(64) void flat_decode_kernel(FlatParams p) {
     const int jr = i16 / p.G;
     const int hq = h * p.G + (i16 - jr * p.G);
     if (i16 < nrows) {
-        const int64_t qoff = (int64_t)(b * p.Sq + jr) * p.q_ts + (int64_t)hq * p.q_hs + 8 * g;
+        const int64_t qoff = (int64_t)(b * p.brows + jr) * p.q_ts + (int64_t)hq * p.q_hs + 8 * g;
 #pragma unroll
         for (int bb = 0; bb < 4; ++bb) qf[bb] = load_q8<QDT>(p.q, qoff + 32 * bb);
         lim = p.q_abs ? min(kvl - 1, p.q_abs[b] + jr) : kvl - 1;
@@ -2605,7 +2708,7 @@ __global__ __launch_bounds__(64) void flat_decode_kernel(FlatParams p) {
     if (i16 >= nrows) return;
     if (p.P == 1) {  // the whole segment: normalized output
         const float inv = l > 0.f ? 1.0f / l : 0.0f;
-        float *ob = p.out + (int64_t)(b * p.Sq + jr) * p.o_ts + (int64_t)hq * p.o_hs + 4 * g;
+        float *ob = p.out + (int64_t)(b * p.brows + jr) * p.o_ts + (int64_t)hq * p.o_hs + 4 * g;
 #pragma unroll
         for (int mm = 0; mm < 8; ++mm) *reinterpret_cast<float4_t *>(ob + 16 * mm) = o[mm] * inv;
     } else {
@@ -2689,7 +2792,7 @@ __global__ __launch_bounds__(FC_THREADS) void flat_combine_kernel(FlatParams p) 
     const int b = seg / p.Hkv, h = seg - b * p.Hkv;
     const int j = r / p.G, hq = h * p.G + (r - j * p.G);
     const float inv = L > 0.f ? 1.0f / L : 0.0f;
-    *reinterpret_cast<float4_t *>(p.out + (int64_t)(b * p.Sq + j) * p.o_ts + (int64_t)hq * p.o_hs + d0) = acc * inv;
+    *reinterpret_cast<float4_t *>(p.out + (int64_t)(b * p.brows + j) * p.o_ts + (int64_t)hq * p.o_hs + d0) = acc * inv;
 }
 
 // ---------------------------------------------------------------------------
@@ -2801,8 +2904,10 @@ void plan_add_class(Plan &pl, int nrg, int lo, int hi) {
 // allow_split: reserve the partial slots of row tiles split over the keys
 // (without them the plan kernel leaves every row tile whole).
 // max_seq_len < 0: unknown (the image room is then the cap).
+// max_pieces: pieces a row tile can be cut into, where the caller knows its
+// longest context for certain (-1: unknown).
 void plan_finish(Plan &pl, int num_seqs, int64_t num_tokens, int G, int num_kv_heads, bool force_pf,
-                 bool allow_split, int64_t max_seq_len, int64_t max_query_len) {
+                 bool allow_split, int64_t max_seq_len, int64_t max_query_len, int64_t max_pieces = -1) {
     pl.dec_rows_max = pl.ndc ? pl.dc[pl.ndc - 1].rows_hi : 0;
     // row tiles over all sequences <= sum ceil(n_q * G / R) <= T*G/R + B (R = pf_rows)
     const int pf_seqs = min(num_seqs, PL_MAX_SEQS);
@@ -2818,6 +2923,7 @@ void plan_finish(Plan &pl, int num_seqs, int64_t num_tokens, int G, int num_kv_h
     pl.pf_items_max = pf ? (int)min(items, (int64_t)INT32_MAX) : 0;
     pl.pf_split_max = pf && allow_split ? (int)(2 * split) : 0;
     pl.pf_slots_max = pf && allow_split ? (int)(3 * split) : 0;
+    if (max_pieces >= 0 && items * max_pieces < pl.pf_slots_max) pl.pf_slots_max = (int)(items * max_pieces);
     pl.pf_grid_items = (int)min(grid_items, (int64_t)INT32_MAX);
     size_t off = 0;
     for (int k = 0; k < pl.ndc; ++k) {
@@ -2930,19 +3036,47 @@ Plan bound_plan(int max_num_seqs, int64_t max_num_tokens, int num_heads, int num
     return pl;
 }
 
+// The plan kernel of a prefill launch with a work list.
+void launch_plan(const AttnParams &p, const Plan &pl, int num_seqs, hipStream_t stream) {
+    // one wave for small batches: its scans and reductions need no
+    // barriers across 16 waves (8 x (32768 + 12) at 48/8: 18.6 us with
+    // 1024 threads)
+    if (num_seqs <= 64 && pl.pf_items_max <= 64) prefill_plan_kernel<64><<<1, 64, 0, stream>>>(p);
+    else prefill_plan_kernel<PL_THREADS><<<1, PL_THREADS, 0, stream>>>(p);
+}
+
+// The workspace's prefill regions (no tile images).
+void set_prefill_ws(AttnParams &p, const Plan &pl, char *ws) {
+    const bool list = pl.pf_items_max > 0;
+    const int ni = pl.pf_grid_items;
+    p.pf_rows = pl.pf_rows;
+    p.pf_items_max = pl.pf_items_max;
+    p.pf_grid_items = ni;
+    p.pf_ncu = device_cus();
+    p.pf_split_max = pl.pf_split_max;
+    p.pf_slots_max = pl.pf_slots_max;
+    p.pf_count = list ? reinterpret_cast<int *>(ws + pl.off_items) : nullptr;
+    p.pf_seq = list ? reinterpret_cast<int *>(ws + pl.off_items + 256) : nullptr;
+    p.pf_rt = list ? p.pf_seq + ni : nullptr;
+    p.pf_kt0 = list ? p.pf_seq + 2 * ni : nullptr;
+    p.pf_kt1 = list ? p.pf_seq + 3 * ni : nullptr;
+    p.pf_slot = list ? p.pf_seq + 4 * ni : nullptr;
+    p.pf_split = list ? reinterpret_cast<int *>(ws + pl.off_split) : nullptr;
+    p.pf_ml = list ? reinterpret_cast<float *>(ws + pl.off_pml) : nullptr;
+    p.pf_o = list ? reinterpret_cast<float *>(ws + pl.off_po) : nullptr;
+    p.pf_tbase = list ? reinterpret_cast<int *>(ws + pl.off_tbase) : nullptr;
+    p.pf_tiles = nullptr;
+    p.pf_tiles_cap = 0;
+    p.pf_img_seq = 0;
+}
+
 template <int QDT, int ODT>
 hipError_t launch_all(const AttnParams &p0, const Plan &pl, char *ws, int num_seqs, int num_kv_heads,
                       int max_query_len, hipStream_t stream) {
     AttnParams p = p0;
     p.dec_rows_lo = 0;
     p.dec_rows_max = pl.dec_rows_max;
-    if (pl.need_prefill && p.pf_seq) {
-        // one wave for small batches: its scans and reductions need no
-        // barriers across 16 waves (8 x (32768 + 12) at 48/8: 18.6 us with
-        // 1024 threads)
-        if (num_seqs <= 64 && pl.pf_items_max <= 64) prefill_plan_kernel<64><<<1, 64, 0, stream>>>(p);
-        else prefill_plan_kernel<PL_THREADS><<<1, PL_THREADS, 0, stream>>>(p);
-    }
+    if (pl.need_prefill && p.pf_seq) launch_plan(p, pl, num_seqs, stream);
     for (int k = 0; k < pl.ndc; ++k) {
         const DecClass &c = pl.dc[k];
         AttnParams pd = p;
@@ -3196,6 +3330,8 @@ hipError_t paged_attention_impl(
     p.bt_stride = block_table_stride;
     p.seq_lens = seq_lens;
     p.qsl = query_start_loc;
+    p.uq = p.uq_rows = 0;
+    p.kv_cap = INT32_MAX;
     p.q_abs = q_abs_offset;
     p.causal = causal ? 1 : 0;
     p.Hkv = num_kv_heads;
@@ -3208,28 +3344,12 @@ hipError_t paged_attention_impl(
     p.o_hs = out_head_stride;
     char *ws = static_cast<char *>(workspace);
     p.num_seqs = num_seqs;
-    p.pf_rows = pl.pf_rows;
-    p.pf_items_max = pl.pf_items_max;
-    p.pf_grid_items = pl.pf_grid_items;
-    p.pf_ncu = device_cus();
-    p.pf_split_max = pl.pf_split_max;
-    p.pf_slots_max = pl.pf_slots_max;
-    const int ni = pl.pf_grid_items;
-    p.pf_count = pl.pf_items_max ? reinterpret_cast<int *>(ws + pl.off_items) : nullptr;
-    p.pf_seq = pl.pf_items_max ? reinterpret_cast<int *>(ws + pl.off_items + 256) : nullptr;
-    p.pf_rt = pl.pf_items_max ? p.pf_seq + ni : nullptr;
-    p.pf_kt0 = pl.pf_items_max ? p.pf_seq + 2 * ni : nullptr;
-    p.pf_kt1 = pl.pf_items_max ? p.pf_seq + 3 * ni : nullptr;
-    p.pf_slot = pl.pf_items_max ? p.pf_seq + 4 * ni : nullptr;
-    p.pf_split = pl.pf_items_max ? reinterpret_cast<int *>(ws + pl.off_split) : nullptr;
-    p.pf_ml = pl.pf_items_max ? reinterpret_cast<float *>(ws + pl.off_pml) : nullptr;
-    p.pf_o = pl.pf_items_max ? reinterpret_cast<float *>(ws + pl.off_po) : nullptr;
+    set_prefill_ws(p, pl, ws);
     // tile images: whatever room the workspace has past the call's regions.
     // None when no sequence can have PF_IMG_REUSE row tiles: the row tiles
     // then read each key tile fewer times than that on average (a sequence's
     // row tiles each read at most the key tiles of its last), so the plan
     // would decline them, and the pre-pass launch is skipped.
-    p.pf_tbase = pl.pf_items_max ? reinterpret_cast<int *>(ws + pl.off_tbase) : nullptr;
     const size_t img_room = workspace_bytes > pl.bytes ? workspace_bytes - pl.bytes : 0;
     const bool img_reuse = pl.pf_rows == PF_ROWS && ((int64_t)max_query_len * G + PF_ROWS - 1) / PF_ROWS >= PF_IMG_REUSE;
     p.pf_tiles = (pl.pf_items_max && img_reuse && img_room >= (size_t)PF_IMG_BYTES)
@@ -3342,6 +3462,13 @@ extern "C" hipError_t gfx906_fa_amd_paged_attention_kv_write(
 
 namespace {
 
+// Masks whose rows start 8-byte aligned and hold whole runs of 4 keys: a
+// lane's four adjacent keys come in one load.
+int mask_vec(const void *mask, int64_t batch_stride, int64_t row_stride, int cols) {
+    return mask != nullptr && ((uintptr_t)mask & 7) == 0 && (batch_stride & 3) == 0 && (row_stride & 3) == 0 &&
+           (cols & 3) == 0;
+}
+
 // Pieces per segment of the contiguous decode: enough single-wave
 // workgroups to fill the device (8 per CU), each at least FD_MIN_SUB
 // sub-pages (its fixed costs - Q load, ring fill, partial write - stay
@@ -3368,30 +3495,25 @@ extern "C" size_t gfx906_fa_amd_flat_decode_workspace_size(int batch, int seq_q,
     return P > 1 ? align256((size_t)nseg * P * rows * FD_ROW * sizeof(float)) : 256;
 }
 
-extern "C" hipError_t gfx906_fa_amd_flat_decode(
-    const void *q, int q_dtype, int64_t q_token_stride, int64_t q_head_stride, const uint8_t *k_q8,
-    const void *v_f16, const int32_t *kv_len, const int32_t *q_abs_offset, int batch, int seq_q, int num_heads,
-    int num_kv_heads, int seq_kv, int head_size, float scale, float *out, int64_t out_token_stride,
-    int64_t out_head_stride, void *workspace, size_t workspace_bytes, hipStream_t stream) {
-    if (batch == 0 || seq_q == 0 || seq_kv == 0) return hipSuccess;
-    const int G = (num_kv_heads > 0 && num_heads > 0) ? num_heads / num_kv_heads : 0;
-    if (head_size != 128 || G <= 0 || num_heads % num_kv_heads || batch < 0 || seq_q < 0 || seq_kv < 0 ||
-        (int64_t)seq_q * G > 16 || q_dtype < 0 || q_dtype > 2 || kv_len == nullptr) {
-        fprintf(stderr, "[gfx906_fa_amd] flat_decode: unsupported configuration (head_size=%d heads=%d/%d seq_q=%d: "
-                        "seq_q * heads/kv_heads must be <= 16; kv_len required)\n",
-                head_size, num_heads, num_kv_heads, seq_q);
-        return hipErrorInvalidValue;
-    }
+namespace {
+
+// Decode shapes over contiguous inputs: brows token rows of q and out per
+// batch row, kv_len may be null (all seq_kv keys).
+hipError_t flat_decode_impl(const char *who, const void *q, int q_dtype, int64_t q_token_stride, int64_t q_head_stride,
+                            const uint8_t *k_q8, const void *v_f16, const int32_t *kv_len, const int32_t *q_abs_offset,
+                            int batch, int seq_q, int brows, int num_heads, int num_kv_heads, int seq_kv, float scale,
+                            float *out, int64_t out_token_stride, int64_t out_head_stride, void *workspace,
+                            size_t workspace_bytes, hipStream_t stream) {
+    const int G = num_heads / num_kv_heads;
     if (((uintptr_t)k_q8 | (uintptr_t)v_f16) & 15u) {
-        fprintf(stderr, "[gfx906_fa_amd] flat_decode: K and V bases must be 16-byte aligned\n");
+        fprintf(stderr, "[gfx906_fa_amd] %s: K and V bases must be 16-byte aligned\n", who);
         return hipErrorInvalidValue;
     }
     const size_t need = gfx906_fa_amd_flat_decode_workspace_size(batch, seq_q, num_heads, num_kv_heads, seq_kv);
     const int nseg = batch * num_kv_heads, nsp = (seq_kv + 15) / 16;
     const int P = flat_pieces(nseg, nsp);
     if (P > 1 && (workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 15u))) {
-        fprintf(stderr, "[gfx906_fa_amd] flat_decode: workspace of %zu bytes required, got %zu\n", need,
-                workspace_bytes);
+        fprintf(stderr, "[gfx906_fa_amd] %s: workspace of %zu bytes required, got %zu\n", who, need, workspace_bytes);
         return hipErrorInvalidValue;
     }
     FlatParams p;
@@ -3409,6 +3531,7 @@ extern "C" hipError_t gfx906_fa_amd_flat_decode(
     p.Skv = seq_kv;
     p.P = P;
     p.nsp = nsp;
+    p.brows = brows;
     p.c = scale * LOG2E;
     p.out = out;
     p.o_ts = out_token_stride;
@@ -3421,6 +3544,128 @@ extern "C" hipError_t gfx906_fa_amd_flat_decode(
         default: flat_decode_kernel<GFA_DTYPE_BF16><<<(unsigned)grid, 64, 0, stream>>>(p); break;
     }
     if (P > 1) flat_combine_kernel<<<dim3(nseg, seq_q * G, FC_DS), FC_THREADS, 0, stream>>>(p);
+    return hipGetLastError();
+}
+
+// Rows per kv-head that the contiguous decode takes (one 16-row group).
+bool flat_is_decode(int seq_q, int G, bool masked) { return !masked && (int64_t)seq_q * G <= 16; }
+
+// The plan of a contiguous attention call past the decode shapes: every batch
+// row is a prefill sequence of seq_q tokens whose tile images are written by
+// the call, in the room past the plan's regions.
+Plan flat_plan(int batch, int seq_q, int num_heads, int num_kv_heads, int seq_kv) {
+    Plan pl{};
+    const int64_t nkt = (seq_kv + PF_TK - 1) / PF_TK;
+    pl.ndc = 0;
+    pl.need_prefill = true;
+    pl.pf_rows = PF_ROWS;
+    plan_finish(pl, batch, (int64_t)batch * seq_q, num_heads / num_kv_heads, num_kv_heads, false, nkt > PF_SPLIT_MIN,
+                seq_kv, 0, (nkt + PF_SPLIT_MIN - 1) / PF_SPLIT_MIN);
+    pl.img_bytes = (size_t)batch * nkt * num_kv_heads * PF_IMG_BYTES;
+    return pl;
+}
+
+}  // namespace
+
+extern "C" hipError_t gfx906_fa_amd_flat_decode(
+    const void *q, int q_dtype, int64_t q_token_stride, int64_t q_head_stride, const uint8_t *k_q8,
+    const void *v_f16, const int32_t *kv_len, const int32_t *q_abs_offset, int batch, int seq_q, int num_heads,
+    int num_kv_heads, int seq_kv, int head_size, float scale, float *out, int64_t out_token_stride,
+    int64_t out_head_stride, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (batch == 0 || seq_q == 0 || seq_kv == 0) return hipSuccess;
+    const int G = (num_kv_heads > 0 && num_heads > 0) ? num_heads / num_kv_heads : 0;
+    if (head_size != 128 || G <= 0 || num_heads % num_kv_heads || batch < 0 || seq_q < 0 || seq_kv < 0 ||
+        (int64_t)seq_q * G > 16 || q_dtype < 0 || q_dtype > 2 || kv_len == nullptr) {
+        fprintf(stderr, "[gfx906_fa_amd] flat_decode: unsupported configuration (head_size=%d heads=%d/%d seq_q=%d: "
+                        "seq_q * heads/kv_heads must be <= 16; kv_len required)\n",
+                head_size, num_heads, num_kv_heads, seq_q);
+        return hipErrorInvalidValue;
+    }
+    return flat_decode_impl("flat_decode", q, q_dtype, q_token_stride, q_head_stride, k_q8, v_f16, kv_len, q_abs_offset,
+                            batch, seq_q, seq_q, num_heads, num_kv_heads, seq_kv, scale, out, out_token_stride,
+                            out_head_stride, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t gfx906_fa_amd_flat_attention_workspace_size(int batch, int seq_q, int num_heads, int num_kv_heads,
+                                                              int seq_kv, int masked) {
+    if (batch <= 0 || seq_q <= 0 || num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads || seq_kv <= 0)
+        return 256;
+    if (flat_is_decode(seq_q, num_heads / num_kv_heads, masked != 0))
+        return gfx906_fa_amd_flat_decode_workspace_size(batch, seq_q, num_heads, num_kv_heads, seq_kv);
+    const Plan pl = flat_plan(batch, seq_q, num_heads, num_kv_heads, seq_kv);
+    return pl.bytes + pl.img_bytes;
+}
+
+extern "C" hipError_t gfx906_fa_amd_flat_attention(
+    const float *q, const uint8_t *k_q8, const void *v_f16, const int32_t *kv_max, const int32_t *q_abs_offset,
+    const void *mask, int64_t mask_batch_stride, int64_t mask_row_stride, int mask_cols, int batch, int seq_q,
+    int num_heads, int num_kv_heads, int seq_kv, int head_size, float scale, float *out, void *workspace,
+    size_t workspace_bytes, hipStream_t stream) {
+    if (batch == 0 || seq_q == 0 || seq_kv == 0) return hipSuccess;
+    const int G = (num_kv_heads > 0 && num_heads > 0) ? num_heads / num_kv_heads : 0;
+    if (head_size != 128 || G <= 0 || num_heads % num_kv_heads || batch < 0 || seq_q < 0 || seq_kv < 0 ||
+        (mask && (mask_cols < 0 || q_abs_offset))) {
+        fprintf(stderr, "[gfx906_fa_amd] flat_attention: unsupported configuration (head_size=%d heads=%d/%d)\n",
+                head_size, num_heads, num_kv_heads);
+        return hipErrorInvalidValue;
+    }
+    const int64_t hs = (int64_t)seq_q * 128;  // q and out: [batch, num_heads, seq_q, 128], contiguous
+    if (flat_is_decode(seq_q, G, mask != nullptr))
+        return flat_decode_impl("flat_attention", q, GFA_DTYPE_F32, 128, hs, k_q8, v_f16, kv_max, q_abs_offset, batch,
+                                seq_q, num_heads * seq_q, num_heads, num_kv_heads, seq_kv, scale, out, 128, hs,
+                                workspace, workspace_bytes, stream);
+    const Plan pl = flat_plan(batch, seq_q, num_heads, num_kv_heads, seq_kv);
+    if (workspace == nullptr || workspace_bytes < pl.bytes + pl.img_bytes || ((uintptr_t)workspace & 255u)) {
+        fprintf(stderr, "[gfx906_fa_amd] flat_attention: workspace of %zu bytes (256-aligned) required, got %zu\n",
+                pl.bytes + pl.img_bytes, workspace_bytes);
+        return hipErrorInvalidValue;
+    }
+    char *ws = static_cast<char *>(workspace);
+    AttnParams p = {};
+    p.q = q;
+    p.q_ts = p.o_ts = 128;
+    p.q_hs = p.o_hs = hs;
+    p.uq = seq_q;
+    p.uq_rows = num_heads * seq_q;
+    p.seq_lens = kv_max;
+    p.kv_cap = seq_kv;
+    p.q_abs = q_abs_offset;
+    p.causal = q_abs_offset != nullptr;
+    p.mask = static_cast<const uint16_t *>(mask);
+    p.mask_bs = mask_batch_stride;
+    p.mask_rs = mask_row_stride;
+    p.mask_cols = mask_cols;
+    p.mask_vec = mask_vec(mask, mask_batch_stride, mask_row_stride, mask_cols);
+    p.Hkv = num_kv_heads;
+    p.G = G;
+    p.block_size = 16;
+    p.scale_log2e = scale * LOG2E;
+    set_prefill_scale(p);
+    p.out = out;
+    p.num_seqs = batch;
+    p.dec_rows_max = 0;  // every batch row through the tiled kernel
+    set_prefill_ws(p, pl, ws);
+    const int nkt = (seq_kv + PF_TK - 1) / PF_TK;
+    p.pf_tiles = reinterpret_cast<uint8_t *>(ws + pl.bytes);
+    p.pf_img_seq = nkt;
+    FlatTiles ft;
+    ft.k = k_q8;
+    ft.v = static_cast<const uint8_t *>(v_f16);
+    ft.img = p.pf_tiles;
+    ft.Hkv = num_kv_heads;
+    ft.Skv = seq_kv;
+    ft.nkt = nkt;
+    ft.k8 = ((uintptr_t)k_q8 & 7u) == 0;
+    ft.v16 = ((uintptr_t)v_f16 & 15u) == 0;
+    ft.kmul = p.pf_kmul;
+    flat_tiles_kernel<<<(unsigned)((int64_t)batch * nkt * num_kv_heads), 256, 0, stream>>>(ft);
+    if (p.pf_seq) launch_plan(p, pl, batch, stream);
+    const int tiles = (int)(((int64_t)seq_q * G + PF_ROWS - 1) / PF_ROWS);
+    const dim3 grid = p.pf_seq ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, batch);
+    if (mask) attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+    else attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+    if (p.pf_seq && pl.pf_slots_max)
+        attn_prefill_combine_kernel<GFA_DTYPE_F32><<<device_cus() * GFA_PFC_WGS_PER_CU, 256, 0, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -3462,14 +3707,14 @@ extern "C" hipError_t gfx906_fa_amd_paged_attention_tiled(
     p.bt_stride = block_table_stride;
     p.seq_lens = seq_lens;
     p.qsl = query_start_loc;
+    p.kv_cap = INT32_MAX;
     p.q_abs = q_abs_offset;
     p.causal = causal ? 1 : 0;
     p.mask = static_cast<const uint16_t *>(mask);
     p.mask_bs = mask_batch_stride;
     p.mask_rs = mask_row_stride;
     p.mask_cols = mask_cols;
-    p.mask_vec = mask != nullptr && ((uintptr_t)mask & 7) == 0 && (mask_batch_stride & 3) == 0 &&
-                 (mask_row_stride & 3) == 0 && (mask_cols & 3) == 0;
+    p.mask_vec = mask_vec(mask, mask_batch_stride, mask_row_stride, mask_cols);
     p.Hkv = num_kv_heads;
     p.G = num_heads / num_kv_heads;
     p.block_size = block_size;

@@ -93,6 +93,8 @@ def _load():
         "gfx906_fa_amd_flat_decode_workspace_size": (SZ, [I, I, I, I, I]),
         "gfx906_fa_amd_flat_decode": (I, [P, I, I64, I64, P, P, P, P, I, I, I, I, I, I, F, P, I64, I64,
                                           P, SZ, P]),
+        "gfx906_fa_amd_flat_attention_workspace_size": (SZ, [I, I, I, I, I, I]),
+        "gfx906_fa_amd_flat_attention": (I, [P, P, P, P, P, P, I64, I64, I, I, I, I, I, I, I, F, P, P, SZ, P]),
         "gfx906_fa_amd_paged_attention_tiled": (I, [P, I, I64, I64, P, P, I, I64, I64, I64, I64, P, I64,
                                                     P, P, P, I, P, I64, I64, I, I, I, I, I, I, I, I,
                                                     F, P, I64, I64, P]),
@@ -575,9 +577,9 @@ def forward(q: torch.Tensor, k_q8: torch.Tensor, v_fp16: torch.Tensor, scale: fl
     only, as the reference launcher (``extension/gfx906_fa_launcher.cu:76-79``).
 
     Decode shapes (Sq * Hq / Hkv <= 16 rows per kv-head, no mask) read K and
-    V in these layouts directly, split over the keys across the device
-    (gfx906_fa_amd_flat_decode); other shapes repack K and V into the planar
-    sub-pages once per call and run the tiled prefill kernel."""
+    V in these layouts directly, split over the keys across the device; other
+    shapes dequantize K and V once per call into tile images and run the tiled
+    prefill kernel over them, long row tiles split over the keys."""
     for t, n in ((q, "q"), (k_q8, "k_q8"), (v_fp16, "v_fp16")):
         _cuda(t, n)
         _check(t.is_contiguous(), f"{n} must be contiguous")
@@ -599,52 +601,27 @@ def forward(q: torch.Tensor, k_q8: torch.Tensor, v_fp16: torch.Tensor, scale: fl
     _check(mask is None or mask.dim() != 3 or mask.shape[2] >= Skv, "mask.size(2) must be >= seq_kv")
     mk, mbs, mrs, mcols = _mask_args(mask, B, Sq, q_abs_offset)
     dev = q.device
-    out = torch.empty((B * Sq, Hq, D), dtype=torch.float32, device=dev)
+    out = torch.empty((B, Hq, Sq, D), dtype=torch.float32, device=dev)
     if B == 0 or Sq == 0 or Hq == 0:
-        return out.view(B, Sq, Hq, D).transpose(1, 2).contiguous()
+        return out
     if kv_max is not None:
         _cuda(kv_max, "kv_max")
         _check(kv_max.dtype == torch.int32, "kv_max must be int32")
         _check(kv_max.dim() == 1 and kv_max.shape[0] == B, "kv_max must be 1D [B]")
-        sl = kv_max.clamp(0, Skv).to(torch.int32).contiguous()
-    else:
-        sl = torch.full((B,), Skv, dtype=torch.int32, device=dev)
+        kv_max = kv_max.contiguous()
     if q_abs_offset is not None:
         _cuda(q_abs_offset, "q_abs_offset")
         _check(q_abs_offset.dtype == torch.int32 and q_abs_offset.dim() == 1 and q_abs_offset.shape[0] == B,
                "q_abs_offset must be 1D [B]")
         q_abs_offset = q_abs_offset.contiguous()
+    if Skv == 0:  # no key: every row is 0
+        return out.zero_()
     L = _load()
-    st = _stream(dev)
-    if mask is None and Sq * (Hq // Hkv) <= 16 and Skv > 0:
-        # decode shapes: the contiguous layouts read as they are, split over the keys
-        q_bshd = q.transpose(1, 2).contiguous().view(B * Sq, Hq, D)
-        ws = new_workspace(L.gfx906_fa_amd_flat_decode_workspace_size(B, Sq, Hq, Hkv, Skv), dev)
-        _ok(L.gfx906_fa_amd_flat_decode(_ptr(q_bshd), _DT[torch.float32], q_bshd.stride(0), q_bshd.stride(1),
-                                         _ptr(k_q8), _ptr(v_fp16), _ptr(sl), _ptr(q_abs_offset), B, Sq, Hq, Hkv,
-                                         Skv, D, float(scale), _ptr(out), out.stride(0), out.stride(1),
-                                         _ptr(ws), ws.numel(), st), "gfx906_fa_amd_flat_decode")
-        return out.view(B, Sq, Hq, D).transpose(1, 2).contiguous()
-    skp = (max(Skv, 1) + SUBPAGE_TOKENS - 1) // SUBPAGE_TOKENS
-    kp = torch.empty((B, Hkv, skp * SUBPAGE_BYTES), dtype=torch.uint8, device=dev)
-    vp = torch.empty((B, Hkv, skp * 4096), dtype=torch.uint8, device=dev)
-    if Skv > 0:
-        _ok(L.gfx906_fa_amd_pack_flat_kv(_ptr(k_q8), _ptr(v_fp16), _ptr(kp), _ptr(vp), B * Hkv, Skv, D, st),
-            "gfx906_fa_amd_pack_flat_kv")
-    else:
-        kp.zero_()
-        vp.zero_()
-    bt = torch.arange(B, dtype=torch.int32, device=dev).view(B, 1)
-    qsl = torch.arange(0, (B + 1) * Sq, Sq, dtype=torch.int32, device=dev)
-    q_bshd = q.transpose(1, 2).contiguous().view(B * Sq, Hq, D)
-    err = L.gfx906_fa_amd_paged_attention_tiled(
-        _ptr(q_bshd), _DT[torch.float32], q_bshd.stride(0), q_bshd.stride(1), _ptr(kp), _ptr(vp), 1,
-        kp.stride(0), kp.stride(1), vp.stride(0), vp.stride(1), _ptr(bt), 1, _ptr(sl), _ptr(qsl),
-        _ptr(q_abs_offset), 1 if q_abs_offset is not None else 0, _ptr(mk), mbs, mrs, mcols,
-        B, B * Sq, Hq, Hkv, D, skp * SUBPAGE_TOKENS, Sq, float(scale), _ptr(out), out.stride(0),
-        out.stride(1), st)
-    _ok(err, "gfx906_fa_amd_paged_attention_tiled")
-    return out.view(B, Sq, Hq, D).transpose(1, 2).contiguous()
+    ws = new_workspace(L.gfx906_fa_amd_flat_attention_workspace_size(B, Sq, Hq, Hkv, Skv, mk is not None), dev)
+    _ok(L.gfx906_fa_amd_flat_attention(_ptr(q), _ptr(k_q8), _ptr(v_fp16), _ptr(kv_max), _ptr(q_abs_offset), _ptr(mk),
+                                       mbs, mrs, mcols, B, Sq, Hq, Hkv, Skv, D, float(scale), _ptr(out), _ptr(ws),
+                                       ws.numel(), _stream(dev)), "gfx906_fa_amd_flat_attention")
+    return out
 
 
 def forward_paged_direct(q: torch.Tensor, key_cache_q8: torch.Tensor, value_cache: torch.Tensor,

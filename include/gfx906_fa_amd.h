@@ -405,6 +405,29 @@ hipError_t gfx906_fa_amd_flat_decode(
     int num_kv_heads, int seq_kv, int head_size, float scale, float *out, int64_t out_token_stride,
     int64_t out_head_stride, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* (8) Contiguous attention in one call (gfx906_fa_launch,
+ *     extension/gfx906_fa_launcher.cu:53-209; gfx906_fa.forward): q and out
+ *     fp32 [batch][num_heads][seq_q][128], k_q8 AoS Q8_0 rows
+ *     [batch][num_kv_heads][seq_kv][136 B], v_f16 fp16 rows
+ *     [batch][num_kv_heads][seq_kv][128], all contiguous.  kv_max int32
+ *     [batch] or NULL (clamped to [0, seq_kv]; NULL: all seq_kv keys),
+ *     q_abs_offset int32 [batch] or NULL (row j sees keys
+ *     k <= q_abs_offset[b] + j), mask NULL or fp16 [batch][seq_q][mask_cols]
+ *     as in (7), exclusive with q_abs_offset.  Decode shapes (no mask,
+ *     seq_q * num_heads / num_kv_heads <= 16) run as flat_decode, K and V
+ *     16-byte aligned; others dequantize K and V once into tile images in the
+ *     workspace (any alignment) and run the tiled kernel over them, long row
+ *     tiles split over the keys.  workspace:
+ *     gfx906_fa_amd_flat_attention_workspace_size() bytes, 256-byte aligned,
+ *     no initial contents. */
+size_t gfx906_fa_amd_flat_attention_workspace_size(int batch, int seq_q, int num_heads, int num_kv_heads,
+                                                   int seq_kv, int masked);
+hipError_t gfx906_fa_amd_flat_attention(
+    const float *q, const uint8_t *k_q8, const void *v_f16, const int32_t *kv_max, const int32_t *q_abs_offset,
+    const void *mask, int64_t mask_batch_stride, int64_t mask_row_stride, int mask_cols, int batch, int seq_q,
+    int num_heads, int num_kv_heads, int seq_kv, int head_size, float scale, float *out, void *workspace,
+    size_t workspace_bytes, hipStream_t stream);
+
 /* Measurement helper: streams `bytes` (a multiple of 16) from the 16-byte
  * aligned device buffer `src` with non-temporal 16-byte loads and writes one
  * XOR word per wave to `out` (at least gfx906_fa_amd_stream_read_words()
