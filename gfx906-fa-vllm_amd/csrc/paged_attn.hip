@@ -56,6 +56,34 @@ constexpr float LOG2E = 1.4426950408889634f;
 #endif
 constexpr int DEC_DEPTH = GFA_DEC_DEPTH;  // decode sub-page ring depth (DEPTH-1 in flight)
 
+// Division of 0 <= n < 2^31 by a launch constant: a high multiply, an add and
+// a shift (exact, Granlund and Montgomery 1994) instead of the compiler's
+// division sequence, which costs a workgroup's start a few hundred cycles.
+struct FastDiv {
+    uint32_t m, l;
+};
+__device__ __forceinline__ int fdiv(int n, FastDiv d) {
+    return (int)((__umulhi((uint32_t)n, d.m) + (uint32_t)n) >> d.l);
+}
+inline FastDiv make_fastdiv(int d) {
+    uint32_t l = 0;
+    while (((uint64_t)1 << l) < (uint64_t)d) ++l;
+    return FastDiv{(uint32_t)((((((uint64_t)1 << l) - (uint64_t)d) << 32) / (uint64_t)d) + 1), l};
+}
+
+// A prefill work item: key tiles [kt0, kt1) of row tile rt of sequence s, and
+// the sequence's scalars (first token row, query tokens, keys, causal offset),
+// so that a workgroup's start is one load deep instead of two.  slot >= 0: a
+// piece of a split row tile, whose partial (m, l, O) goes to that partial
+// slot (merged by attn_prefill_combine_kernel); else the piece is the whole
+// row tile and writes the output.
+struct __attribute__((aligned(16))) PfItem {
+    int s, rt, kt0, kt1;
+    int slot, q0, nq, sl;
+    int qa, pad[3];
+};
+static_assert(sizeof(PfItem) == 48, "three 16-byte loads");
+
 struct AttnParams {
     const void *q;
     int64_t q_ts, q_hs;
@@ -87,14 +115,12 @@ struct AttnParams {
     int dec_rows_lo;      // a decode launch takes sequences with dec_rows_lo < n_q*G
     int dec_rows_max;     //   <= dec_rows_max; the prefill kernel takes n_q*G > dec_rows_max
                           //   (in a decode launch also the rows of its partial slots)
-    // prefill work list (heaviest first) built by prefill_plan_kernel: item i
-    // is key tiles [pf_kt0[i], pf_kt1[i]) of row tile pf_rt[i] of sequence
-    // pf_seq[i], *pf_count items; pf_slot[i] >= 0: a piece of a split row
-    // tile, whose partial (m, l, O) goes to partial slot pf_slot[i] (merged
-    // by attn_prefill_combine_kernel), else the piece is the whole row tile
-    // and writes the output.  nullptr: the prefill grid is
-    // (row tiles * Hkv, num_seqs) instead, with no split.
-    int *pf_seq, *pf_rt, *pf_kt0, *pf_kt1, *pf_slot, *pf_count;
+    // prefill work list (heaviest first) built by prefill_plan_kernel,
+    // *pf_count items.  nullptr: the prefill grid is (row tiles * Hkv,
+    // num_seqs) instead, with no split.
+    PfItem *pf_items;
+    int *pf_count;
+    FastDiv g_div, spp_div;  // by G; by sub-pages per page
     int pf_rows;        // query rows per prefill row tile: PF_ROWS, or PF_ROWS / 2 (KS = 2 tiles)
     int pf_items_max;   // row tiles, at most
     int pf_grid_items;  // work-list capacity (the grid): row tiles + extra pieces
@@ -163,6 +189,17 @@ __device__ __forceinline__ void store_out(void *out, int64_t off, float v) {
         const uint32_t u = __float_as_uint(v);
         const uint32_t r = (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
         static_cast<uint16_t *>(out)[off] = (uint16_t)r;
+    }
+}
+
+// Two outputs as they lie next to each other in memory (16-bit types).
+template <int ODT>
+__device__ __forceinline__ uint32_t pack2_out(float a, float b) {
+    if constexpr (ODT == GFA_DTYPE_F16) {
+        return (uint32_t)__builtin_bit_cast(uint16_t, (half_t)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (half_t)b) << 16);
+    } else {
+        const uint32_t u = __float_as_uint(a), v = __float_as_uint(b);
+        return ((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16) | ((v + 0x7FFFu + ((v >> 16) & 1u)) & 0xFFFF0000u);
     }
 }
 
@@ -1187,6 +1224,8 @@ constexpr int PF_KPITCH = 272;
 constexpr int PF_VPITCH = 2 * PF_TK + 16;
 constexpr int PF_KBYTES = PF_TK * PF_KPITCH;
 constexpr int PF_VBYTES = 128 * PF_VPITCH;
+constexpr int PF_QBYTES = 32 * PF_KPITCH;            // a consumer wave's Q rows in LDS, fp16
+static_assert(4 * PF_QBYTES <= 2 * PF_KBYTES && 4 * PF_QBYTES <= 2 * PF_VBYTES, "Q rows fit two stages");
 constexpr int PF_IMG_BYTES = PF_KBYTES + PF_VBYTES;  // one tile image: K^ stage, then V^T stage
 constexpr int PF_NSTAGE = 3;                           // LDS stages of K^ and of V^T (tile t: stage t % 3)
 #ifndef GFA_PF_IMG_REUSE
@@ -1334,43 +1373,51 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
     static_assert(KS == 1 || KS == 2, "256-row tiles, or 128-row key-interleaved tiles");
     constexpr int ROWS = PF_ROWS / KS;               // query rows per tile
     constexpr int NSTAGE = KS == 1 ? PF_NSTAGE : 2;  // LDS stages of K^ and of V^T (tile t: t % NSTAGE)
-    __shared__ __attribute__((aligned(16))) uint8_t lds[NSTAGE * (PF_KBYTES + PF_VBYTES)];
+    // (KS = 2 has room for the consumers' Q rows of its own; KS = 1 puts them
+    // into the stages 1 and 2, free until the first tile has been written)
+    constexpr int STAGES = NSTAGE * (PF_KBYTES + PF_VBYTES);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[STAGES + (KS == 2 ? PF_CWAVES * PF_QBYTES : 0)];
     uint8_t *const ldsk = lds;
     uint8_t *const ldsv = lds + NSTAGE * PF_KBYTES;
     const int Hkv = p.Hkv;
     const int h = blockIdx.x % Hkv;
-    int s, rt, kt0 = 0, kt1 = INT32_MAX, slot = -1;
-    if (p.pf_seq) {  // the sorted work list (uniform)
+    PfItem it;
+    if (p.pf_items) {  // the sorted work list (uniform)
         const int item = blockIdx.x / Hkv;
+        it = p.pf_items[item];  // (in flight together with the count)
         if (item >= p.pf_count[0]) return;
-        s = p.pf_seq[item];
-        rt = p.pf_rt[item];
-        kt0 = p.pf_kt0[item];
-        kt1 = p.pf_kt1[item];
-        slot = p.pf_slot[item];
-    } else {         // row tiles last-first within each sequence
-        s = blockIdx.y;
-        rt = (gridDim.x / Hkv) - 1 - (int)(blockIdx.x / Hkv);
+    } else {           // row tiles last-first within each sequence
+        it.s = blockIdx.y;
+        it.rt = (gridDim.x / Hkv) - 1 - (int)(blockIdx.x / Hkv);
+        it.kt0 = 0;
+        it.kt1 = INT32_MAX;
+        it.slot = -1;
+        it.q0 = seq_q0(p, it.s);
+        it.nq = seq_nq(p, it.s);
+        it.sl = seq_len(p, it.s);
+        it.qa = p.q_abs ? p.q_abs[it.s] : it.sl - it.nq;
     }
-    const int q0 = seq_q0(p, s);
-    const int nq = seq_nq(p, s);
+    const int s = it.s, rt = it.rt, kt0 = it.kt0, kt1 = it.kt1, slot = it.slot;
+    const int q0 = it.q0, nq = it.nq, sl = it.sl, qa = it.qa;
     const int nrows = nq * p.G;
     if (nq <= 0 || nrows <= p.dec_rows_max) return;  // uniform over the workgroup
     const int row0 = ROWS * rt;
     if (row0 >= nrows) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int sl = seq_len(p, s);
-    const int qa = p.q_abs ? p.q_abs[s] : sl - nq;
-    const int jlast = (min(row0 + ROWS, nrows) - 1) / p.G;
+    const int jlast = fdiv(min(row0 + ROWS, nrows) - 1, p.g_div);
     const int kv_end = p.causal ? min(sl, max(qa + jlast + 1, 0)) : sl;
     // key tiles [ktb, ktb + ntk) of the row tile's (kv_end + PF_TK - 1) / PF_TK;
     // the loops below count tiles from 0 and add ktb where they need a key index
     const int ntk_all = (kv_end + PF_TK - 1) / PF_TK;
     const int ktb = min(kt0, ntk_all);
     const int ntk = min(kt1, ntk_all) - ktb;
-    using Even = std::integral_constant<bool, false>;
-    using Odd = std::integral_constant<bool, true>;
+    // The consumers' Q loads would hold up the producers' page ids and first
+    // tile in the CU's memory pipeline, so the consumers wait at this barrier
+    // until those are issued (a bare s_barrier: nothing in flight is waited
+    // for).  A producer's page ids then come 0.4 us after its work item
+    // instead of 2.1 to 3.3 us.
+    auto first_loads_issued = []() __attribute__((always_inline)) { __builtin_amdgcn_s_barrier(); };
 
     if (w >= PF_CWAVES) {
         // ---- producer: sub-page wsp of every tile, both halves ----------
@@ -1410,15 +1457,18 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
                     __builtin_amdgcn_global_load_lds(src + 4096 + lane * 16,
                                                      (__attribute__((address_space(3))) void *)(dst + 4096), 16, 0, 0);
             };
-            // the end of half-step h (h = -1: before the first barrier)
+            // the end of half-step h
             auto landed = [&](int h) __attribute__((always_inline)) {
                 if (h + 4 < 2 * ntk) __builtin_amdgcn_s_waitcnt(0x0F7F);  // vmcnt(15)
                 else __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
             };
-#pragma unroll
-            for (int b = 0; b < 4; ++b) copy(b);
-            landed(-1);
+            copy(0);
+            first_loads_issued();
+            copy(1);
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             __syncthreads();
+            copy(2);  // (stage 1 held Q rows before)
+            copy(3);
             for (int hs = 0; hs <= 2 * ntk; ++hs) {  // half-steps 0 .. 2 ntk
                 copy(hs + 4);
                 landed(hs);
@@ -1427,13 +1477,17 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             return;
         }
         const int32_t *btrow = p.bt + (int64_t)s * p.bt_stride;
-        const int bs = p.block_size;
+        const int spp = p.block_size >> 4;              // sub-pages per page
         const int last_sp = max((kv_end - 1) >> 4, 0);  // last sub-page with a valid key
         const int spb = PF_NSP * ktb + wsp;
-        auto sp_of = [&](int kt) { return min(PF_NSP * kt + spb, last_sp); };
-        auto load_pg = [&](int c) -> int {
+        // the page of this wave's sub-page of tile 64 c + lane, and the
+        // sub-page's index in it
+        auto load_pg = [&](int c, int &spi) __attribute__((always_inline)) -> int {
             const int kt = 64 * c + lane;
-            return kt < ntk ? btrow[(16 * sp_of(kt)) / bs] : 0;
+            const int sp = min(PF_NSP * kt + spb, last_sp);
+            const int pi = fdiv(sp, p.spp_div);
+            spi = sp - pi * spp;
+            return kt < ntk ? btrow[pi] : 0;
         };
         // Waits for a window load right where it is issued (once per 64
         // tiles): a window register still pending in the loop would make
@@ -1443,7 +1497,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
         const uint8_t *kplane = p.kc + (int64_t)h * p.chs;
         const uint8_t *vplane = p.vc + (int64_t)h * p.vchs;
         constexpr int VSUB = VF16 ? 4096 : SUBPAGE_BYTES;  // V bytes per 16-token sub-page
-        int pw0 = 0, pw1 = 0, cbase = 0;
+        int pw0 = 0, pw1 = 0, ps0 = 0, ps1 = 0, cbase = 0;
         struct PfRawT {
             PfRaw h[2];
         };
@@ -1458,8 +1512,10 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             const int rel = t - cbase;  // 0..127, uniform
             const int pa = __builtin_amdgcn_readlane(pw0, rel & 63);
             const int pb = __builtin_amdgcn_readlane(pw1, rel & 63);
+            const int sa = __builtin_amdgcn_readlane(ps0, rel & 63);
+            const int sb = __builtin_amdgcn_readlane(ps1, rel & 63);
             const int64_t page = rel < 64 ? pa : pb;
-            const int64_t spi = ((16 * sp_of(t)) % bs) >> 4;
+            const int64_t spi = rel < 64 ? sa : sb;
             const uint8_t *kb = kplane + page * p.cbs + spi * SUBPAGE_BYTES;
             const uint8_t *vb = vplane + page * p.vcbs + spi * VSUB;
             pf_fetch<VF16>(rw.h[0], kb, vb, lane, 0);
@@ -1472,7 +1528,8 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             if (kt - cbase >= 64) {
                 cbase += 64;
                 pw0 = pw1;
-                pw1 = cbase + 64 < ntk ? load_pg(cbase / 64 + 1) : 0;
+                ps0 = ps1;
+                pw1 = cbase + 64 < ntk ? load_pg(cbase / 64 + 1, ps1) : 0;
                 ready(pw1);
             }
         };
@@ -1503,13 +1560,17 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             // of tile h its ring slot takes tile h + PF_PDEPTH.
             static_assert(KS != 2 || PF_PDEPTH == 4, "the KS = 2 producer loop is unrolled for a 4-deep ring");
             if (ntk > 0) {
-                pw0 = load_pg(0);
-                pw1 = ntk > 64 ? load_pg(1) : 0;
+                pw0 = load_pg(0, ps0);
+                pw1 = ntk > 64 ? load_pg(1, ps1) : 0;
                 ready(pw0);
                 ready(pw1);
+                fetch(ring[0], 0);
+                first_loads_issued();
 #pragma unroll
-                for (int i = 0; i < PF_PDEPTH; ++i) fetch(ring[i], i);
+                for (int i = 1; i < PF_PDEPTH; ++i) fetch(ring[i], i);
                 dequant_k(ring[0], 0);
+            } else {
+                first_loads_issued();
             }
             __syncthreads();
             // a half-step h < ntk - 1: tile h + 1 in slot SK, tile h in slot SV
@@ -1548,16 +1609,20 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             return;
         }
         if (ntk > 0) {
-            pw0 = load_pg(0);
-            pw1 = ntk > 64 ? load_pg(1) : 0;
+            pw0 = load_pg(0, ps0);
+            pw1 = ntk > 64 ? load_pg(1, ps1) : 0;
             ready(pw0);
             ready(pw1);
+            fetch(ring[0], 0);
+            first_loads_issued();
 #pragma unroll
-            for (int i = 0; i < PF_PDEPTH; ++i) fetch(ring[i], i);
+            for (int i = 1; i < PF_PDEPTH; ++i) fetch(ring[i], i);
             dequant_k(ring[0], 0);
             if (ntk == 1) dequant_v(ring[0], 0, IsTail{});
             else dequant_v(ring[0], 0, NoTail{});
             fetch(ring[0], PF_PDEPTH);
+        } else {
+            first_loads_issued();
         }
         __syncthreads();
         // Half-steps h = 0 .. 2 ntk (a barrier each): K^ of tile t is written in
@@ -1607,6 +1672,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
     }
 
     // ---- consumer: 32 query rows ----------------------------------------
+    first_loads_issued();
     const int hb = lane >> 5;
     // the wave's 32-row chunk of the tile and its group (A: 0, B: 1)
     const int cw = KS == 1 ? w : w % (PF_CWAVES / 2);
@@ -1614,7 +1680,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
     // this lane's query row, its causal bound and its Q^T fragments
     const int r = row0 + 32 * cw + (lane & 31);
     const bool rvalid = r < nrows;
-    const int j = rvalid ? r / p.G : 0;
+    const int j = rvalid ? fdiv(r, p.g_div) : 0;
     const int hq = h * p.G + (rvalid ? r - j * p.G : 0);
     const int lim = rvalid ? (p.causal ? min(sl - 1, qa + j) : sl - 1) : INT32_MAX;
     const bool wact = row0 + 32 * cw < nrows;  // uniform over the wave (and its KS = 2 partner)
@@ -1624,17 +1690,39 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
         for (int i = 0; i < (KS == 1 ? 2 * ntk + 2 : ntk + 3); ++i) __syncthreads();
         return;
     }
+    // Q^T fragments (lane: its row, 8 d of every 16).  Loaded straight into
+    // that layout, each of a workgroup's 64 load instructions touched 32 rows;
+    // instead 16 lanes read a whole row (4 rows an instruction) and the wave
+    // turns the fp16 rows over through LDS.  First QK after a workgroup's
+    // start, 48/8 heads, 42-token chunks: 4.7 -> 4.0 us with one workgroup
+    // per kv-head, 6.0 -> 5.4 us with the device full (then the first reads
+    // of all workgroups together, 26 MB, set the time).
     half8_t qf[8];
     {
         const float c = p.pf_qmul;  // a power of two: exact for fp16 / bf16 Q
-        const int64_t qoff = (int64_t)(q0 + j) * p.q_ts + (int64_t)hq * p.q_hs + 8 * hb;
+        const int64_t qrow = (int64_t)(q0 + j) * p.q_ts + (int64_t)hq * p.q_hs;  // (rows past nrows: row j = 0)
+        uint8_t *const ql = KS == 2 ? lds + STAGES + w * PF_QBYTES
+                                    : (w < 4 ? ldsk + PF_KBYTES : ldsv + PF_VBYTES) + (w & 3) * PF_QBYTES;
+        half8_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int src = 4 * i + (lane >> 4);
+            const int64_t off = ((int64_t)__shfl((int)(qrow >> 32), src) << 32) + (uint32_t)__shfl((int)qrow, src) +
+                                8 * (lane & 15);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[i][e] = (half_t)(load_as_f32<QDT>(p.q, off + e) * c);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<half8_t *>(ql + (4 * i + (lane >> 4)) * PF_KPITCH + 16 * (lane & 15)) = x[i];
+        // (one wave's LDS instructions complete in order; the fence keeps the
+        // compiler's order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {  // (row j = 0 stands in for rows past nrows: a valid address)
-                const float v = load_as_f32<QDT>(p.q, qoff + 16 * kk + e);
-                qf[kk][e] = rvalid ? (half_t)(v * c) : (half_t)0.0f;
-            }
+            qf[kk] = *reinterpret_cast<const half8_t *>(ql + (lane & 31) * PF_KPITCH + 32 * kk + 16 * hb);
+            if (!rvalid) qf[kk] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
         }
     }
     int lim_min;  // smallest bound over the wave's rows: tiles below it need no mask
@@ -1895,12 +1983,37 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             }
         } else if (rvalid) {
             const float inv = l > 0.f ? 1.0f / l : 0.0f;
-            const int64_t ob = (int64_t)(q0 + j) * p.o_ts + (int64_t)hq * p.o_hs + 4 * hb;
+            const int64_t ob = (int64_t)(q0 + j) * p.o_ts + (int64_t)hq * p.o_hs;
+            if constexpr (ODT == GFA_DTYPE_F32) {
 #pragma unroll
-            for (int dt = DB; dt < DB + ND; ++dt)
+                for (int dt = DB; dt < DB + ND; ++dt)
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    store_out<ODT>(p.out, ob + 32 * dt + 8 * (e >> 2) + (e & 3), o[dt][e] * inv);
+                    for (int e = 0; e < 16; ++e)
+                        store_out<ODT>(p.out, ob + 4 * hb + 32 * dt + 8 * (e >> 2) + (e & 3), o[dt][e] * inv);
+            } else {
+                // 16 bytes per lane: lane l holds d = 8q + 4hb .. + 3 of its
+                // row; of each pair of q the lanes l and l + 32 swap a half, so
+                // that hb = 0 stores the eight d of the even q and hb = 1 those
+                // of the odd one.  A store instruction touches 32 rows either
+                // way, so half as many take half the time of the address unit
+                // (a wave's 16 eight-byte stores took 1.6 us).
+#pragma unroll
+                for (int dt = DB; dt < DB + ND; ++dt)
+#pragma unroll
+                    for (int qp = 0; qp < 2; ++qp) {
+                        u32x4 w;
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {  // dword i of the four values
+                            const uint32_t ev = pack2_out<ODT>(o[dt][8 * qp + 2 * i] * inv, o[dt][8 * qp + 2 * i + 1] * inv);
+                            const uint32_t od =
+                                pack2_out<ODT>(o[dt][8 * qp + 4 + 2 * i] * inv, o[dt][8 * qp + 5 + 2 * i] * inv);
+                            const auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
+                            w[i] = sw[0];
+                            w[2 + i] = sw[1];
+                        }
+                        __builtin_memcpy(static_cast<uint16_t *>(p.out) + ob + 32 * dt + 16 * qp + 8 * hb, &w, 16);
+                    }
+            }
         }
     };
     if constexpr (KS == 1) store_tiles(D0{}, std::integral_constant<int, 4>{});
@@ -2237,6 +2350,8 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
         locate(i, sq, rt);
         const int w = ntk_of(i, sq, rt);
         const int k = pl_pieces(w, tsplit);
+        const PlSeq qs = seq_of(sq);
+        const int q0 = seq_q0(p, sq);
         int slot0 = -1;
         if (k > 1) {
             slot0 = atomicAdd(&s_nslot, k);
@@ -2256,11 +2371,8 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
             b = a + q + (rem >= k ? 1 : 0);
             rem -= rem >= k ? k : 0;
             const int pos = atomicAdd(&s_bk[pl_bucket(b - a)], 1);
-            p.pf_seq[pos] = sq;
-            p.pf_rt[pos] = rt;
-            p.pf_kt0[pos] = a;
-            p.pf_kt1[pos] = k > 1 ? b : INT32_MAX;
-            p.pf_slot[pos] = k > 1 ? slot0 + c : -1;
+            p.pf_items[pos] = PfItem{sq, rt, a, k > 1 ? b : INT32_MAX, k > 1 ? slot0 + c : -1, q0, qs.nq, qs.sl,
+                                     qs.qa, {0, 0, 0}};
         }
     }
     pl_sync<NT>();
@@ -2842,6 +2954,7 @@ struct Plan {
     int pf_slots_max;   // partial slots per kv head
     int pf_grid_items;  // work-list capacity: the prefill grid over Hkv
     size_t off_items, off_split, off_pml, off_po, off_tbase;
+    size_t list_extra;  // bytes of the work list past 20 an item (see the allocation-free entry)
     size_t bytes;       // the regions a call needs; the tile images follow at `bytes`
     size_t img_bytes;   // room the tile images of the call's shape can take (capped)
     bool comb_short;    // contexts of at most GFA_COMB_FEW_KEYS keys (combine choice)
@@ -2868,6 +2981,12 @@ void set_prefill_scale(AttnParams &p) {
     e = max(-60, min(60, -e));
     p.pf_qmul = ldexpf(1.0f, -e);
     p.pf_kmul = ldexpf(p.scale_log2e, e);
+}
+
+// The launch constants the kernels divide by.
+void set_divisors(AttnParams &p) {
+    p.g_div = make_fastdiv(p.G);
+    p.spp_div = make_fastdiv(p.block_size >> 4);
 }
 
 // CUs of the current device, queried once per device.  Threads may race on
@@ -2937,9 +3056,10 @@ void plan_finish(Plan &pl, int num_seqs, int64_t num_tokens, int G, int num_kv_h
     }
     pl.off_items = off;
     // work list: a 256-byte header (item count, split row tile count), the
-    // five item arrays, the split list, then the partials of the split pieces
-    // (slots of the call's tile rows)
-    pl.off_split = pl.off_items + 256 + align256((size_t)5 * grid_items * sizeof(int));
+    // items, the split list, then the partials of the split pieces (slots of
+    // the call's tile rows)
+    pl.off_split = pl.off_items + 256 + align256((size_t)grid_items * sizeof(PfItem));
+    pl.list_extra = align256((size_t)grid_items * sizeof(PfItem)) - align256((size_t)5 * grid_items * sizeof(int));
     // partial slots of the call's tile rows (a bound over every call: PF_ROWS)
     const size_t prow = (size_t)pl.pf_slots_max * num_kv_heads * (force_pf ? PF_ROWS : pl.pf_rows);
     pl.off_pml = pl.off_split + align256((size_t)4 * pl.pf_split_max * sizeof(int));
@@ -3048,19 +3168,14 @@ void launch_plan(const AttnParams &p, const Plan &pl, int num_seqs, hipStream_t 
 // The workspace's prefill regions (no tile images).
 void set_prefill_ws(AttnParams &p, const Plan &pl, char *ws) {
     const bool list = pl.pf_items_max > 0;
-    const int ni = pl.pf_grid_items;
     p.pf_rows = pl.pf_rows;
     p.pf_items_max = pl.pf_items_max;
-    p.pf_grid_items = ni;
+    p.pf_grid_items = pl.pf_grid_items;
     p.pf_ncu = device_cus();
     p.pf_split_max = pl.pf_split_max;
     p.pf_slots_max = pl.pf_slots_max;
     p.pf_count = list ? reinterpret_cast<int *>(ws + pl.off_items) : nullptr;
-    p.pf_seq = list ? reinterpret_cast<int *>(ws + pl.off_items + 256) : nullptr;
-    p.pf_rt = list ? p.pf_seq + ni : nullptr;
-    p.pf_kt0 = list ? p.pf_seq + 2 * ni : nullptr;
-    p.pf_kt1 = list ? p.pf_seq + 3 * ni : nullptr;
-    p.pf_slot = list ? p.pf_seq + 4 * ni : nullptr;
+    p.pf_items = list ? reinterpret_cast<PfItem *>(ws + pl.off_items + 256) : nullptr;
     p.pf_split = list ? reinterpret_cast<int *>(ws + pl.off_split) : nullptr;
     p.pf_ml = list ? reinterpret_cast<float *>(ws + pl.off_pml) : nullptr;
     p.pf_o = list ? reinterpret_cast<float *>(ws + pl.off_po) : nullptr;
@@ -3076,7 +3191,7 @@ hipError_t launch_all(const AttnParams &p0, const Plan &pl, char *ws, int num_se
     AttnParams p = p0;
     p.dec_rows_lo = 0;
     p.dec_rows_max = pl.dec_rows_max;
-    if (pl.need_prefill && p.pf_seq) launch_plan(p, pl, num_seqs, stream);
+    if (pl.need_prefill && p.pf_items) launch_plan(p, pl, num_seqs, stream);
     for (int k = 0; k < pl.ndc; ++k) {
         const DecClass &c = pl.dc[k];
         AttnParams pd = p;
@@ -3120,13 +3235,13 @@ hipError_t launch_all(const AttnParams &p0, const Plan &pl, char *ws, int num_se
         // the tile images, after the decode launches (their write-back then
         // overlaps the MFMA-bound prefill, not the HBM-bound decode); returns
         // at once when the plan chose none
-        if (p.pf_seq && p.pf_tiles) prefill_tiles_kernel<false><<<device_cus() * 4, 64 * PF_NSP, 0, stream>>>(p);
+        if (p.pf_items && p.pf_tiles) prefill_tiles_kernel<false><<<device_cus() * 4, 64 * PF_NSP, 0, stream>>>(p);
         const int rows = max_query_len * p.G;
         const int tiles = (rows + pl.pf_rows - 1) / pl.pf_rows;
-        const dim3 grid = p.pf_seq ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, num_seqs);
+        const dim3 grid = p.pf_items ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, num_seqs);
         if (pl.pf_rows == PF_ROWS) attn_prefill_kernel<QDT, ODT, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
         else attn_prefill_kernel<QDT, ODT, false, false, 2><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
-        if (p.pf_seq && pl.pf_split_max)  // returns at once when the plan split nothing
+        if (p.pf_items && pl.pf_split_max)  // returns at once when the plan split nothing
             attn_prefill_combine_kernel<ODT><<<device_cus() * GFA_PFC_WGS_PER_CU, 256, 0, stream>>>(p);
     }
     return hipGetLastError();
@@ -3300,6 +3415,13 @@ hipError_t paged_attention_impl(
         if (pl.bytes > GFX906_FA_AMD_SCRATCH_BYTES)
             pl = make_plan(num_seqs, num_tokens, num_heads, num_kv_heads, max(max_query_len, 1),
                            max(max_seq_len, 1), false);
+        if (pl.bytes > GFX906_FA_AMD_SCRATCH_BYTES && pl.pf_items_max > 0 &&
+            pl.bytes - pl.list_extra <= GFX906_FA_AMD_SCRATCH_BYTES) {
+            // millions of query tokens, whose work list alone passes the
+            // scratch: the 2-D prefill grid needs none
+            pl.pf_items_max = pl.pf_grid_items = pl.pf_split_max = pl.pf_slots_max = 0;
+            pl.bytes = max(pl.off_items, (size_t)256);
+        }
         if (pl.bytes > GFX906_FA_AMD_SCRATCH_BYTES) {
             fprintf(stderr,
                     "[gfx906_fa_amd] paged_attention_noalloc: this batch needs %zu bytes of scratch, more than "
@@ -3339,6 +3461,7 @@ hipError_t paged_attention_impl(
     p.block_size = block_size;
     p.scale_log2e = scale * LOG2E;
     set_prefill_scale(p);
+    set_divisors(p);
     p.out = out;
     p.o_ts = out_token_stride;
     p.o_hs = out_head_stride;
@@ -3641,6 +3764,7 @@ extern "C" hipError_t gfx906_fa_amd_flat_attention(
     p.block_size = 16;
     p.scale_log2e = scale * LOG2E;
     set_prefill_scale(p);
+    set_divisors(p);
     p.out = out;
     p.num_seqs = batch;
     p.dec_rows_max = 0;  // every batch row through the tiled kernel
@@ -3659,12 +3783,12 @@ extern "C" hipError_t gfx906_fa_amd_flat_attention(
     ft.v16 = ((uintptr_t)v_f16 & 15u) == 0;
     ft.kmul = p.pf_kmul;
     flat_tiles_kernel<<<(unsigned)((int64_t)batch * nkt * num_kv_heads), 256, 0, stream>>>(ft);
-    if (p.pf_seq) launch_plan(p, pl, batch, stream);
+    if (p.pf_items) launch_plan(p, pl, batch, stream);
     const int tiles = (int)(((int64_t)seq_q * G + PF_ROWS - 1) / PF_ROWS);
-    const dim3 grid = p.pf_seq ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, batch);
+    const dim3 grid = p.pf_items ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, batch);
     if (mask) attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
     else attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
-    if (p.pf_seq && pl.pf_slots_max)
+    if (p.pf_items && pl.pf_slots_max)
         attn_prefill_combine_kernel<GFA_DTYPE_F32><<<device_cus() * GFA_PFC_WGS_PER_CU, 256, 0, stream>>>(p);
     return hipGetLastError();
 }
@@ -3720,6 +3844,7 @@ extern "C" hipError_t gfx906_fa_amd_paged_attention_tiled(
     p.block_size = block_size;
     p.scale_log2e = scale * LOG2E;
     set_prefill_scale(p);
+    set_divisors(p);
     p.out = out;
     p.o_ts = out_token_stride;
     p.o_hs = out_head_stride;
