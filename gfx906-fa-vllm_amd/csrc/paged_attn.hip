@@ -2039,24 +2039,9 @@ constexpr int PF_SPLIT_MIN = GFA_PF_SPLIT_MIN;  // a split row tile's pieces: at
 #define GFA_PFC_WGS_PER_CU 4  // split-merge workgroups per CU (more loads in flight)
 #endif
 
-// The plan's workgroup-wide ordering point.  On one wave (NT = 64) it needs
-// no barrier: a wave's LDS instructions complete in the order it issues
-// them, and the wave-scope fence keeps the compiler from moving LDS accesses
-// across it.  (A workgroup barrier would also wait for the wave's global
-// stores to complete, which the plan never needs.)
-template <int NT>
-__device__ __forceinline__ void pl_sync() {
-    if constexpr (NT == 64) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    } else {
-        __syncthreads();
-    }
-}
-
-template <int CTRL>
+template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ int dpp_i32(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
 }
 
 // sum over the wave, every lane receives it: butterflies within each 16-lane
@@ -2072,21 +2057,36 @@ __device__ __forceinline__ int pl_wave_sum32(int v) {
     return (int)(b[0] + b[1]);
 }
 
+// max over the wave, every lane receives it
+__device__ __forceinline__ int pl_wave_max32(int v) {
+    v = max(v, dpp_i32<DPP_QUAD_XOR1>(v));
+    v = max(v, dpp_i32<DPP_QUAD_XOR2>(v));
+    v = max(v, dpp_i32<DPP_ROW_HALF_MIRROR>(v));
+    v = max(v, dpp_i32<DPP_ROW_MIRROR>(v));
+    const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+    v = max((int)a[0], (int)a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    return max((int)b[0], (int)b[1]);
+}
+
+// inclusive scan over the wave: shifts within each 16-lane DPP row, then the
+// rows' totals broadcast to the rows after them
+__device__ __forceinline__ int pl_wave_scan32(int v) {
+    v += dpp_i32<0x111>(v);       // row_shr:1
+    v += dpp_i32<0x112>(v);       // row_shr:2
+    v += dpp_i32<0x114>(v);       // row_shr:4
+    v += dpp_i32<0x118>(v);       // row_shr:8
+    v += dpp_i32<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp_i32<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // exclusive scan of v over the workgroup; *total receives the sum (a scan
 // inside each wave, then the waves' totals through tmp)
-template <int NT>
 __device__ __forceinline__ int pl_block_scan(int v, int *tmp, int *total) {
+    constexpr int NT = PL_THREADS;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(x, off);
-        if (lane >= off) x += y;
-    }
-    if constexpr (NT == 64) {
-        *total = __builtin_amdgcn_readlane(x, 63);
-        return x - v;
-    }
+    const int x = pl_wave_scan32(v);
     __syncthreads();  // tmp[] of a previous call has been read
     if (lane == 63) tmp[wv] = x;
     __syncthreads();
@@ -2142,11 +2142,10 @@ __device__ __forceinline__ int pl_ntk(const AttnParams &p, const PlSeq &q, int r
 __device__ __forceinline__ int pl_bucket(int tiles) { return min(tiles, PL_BUCKETS - 1); }
 
 // sum of v over the workgroup (every thread receives it)
-template <int NT>
 __device__ __forceinline__ long long pl_block_sum(long long v, long long *red) {
+    constexpr int NT = PL_THREADS;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    if constexpr (NT == 64) return uniform64(v);  // (in scalar registers: the plan's control flow is uniform)
     __syncthreads();  // red[] of a previous call has been read
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -2157,11 +2156,10 @@ __device__ __forceinline__ long long pl_block_sum(long long v, long long *red) {
 }
 
 // max of v over the workgroup (every thread receives it)
-template <int NT>
 __device__ __forceinline__ long long pl_block_max(long long v, long long *red) {
+    constexpr int NT = PL_THREADS;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = max(v, (long long)__shfl_xor(v, off));
-    if constexpr (NT == 64) return uniform64(v);
     __syncthreads();  // red[] of a previous call has been read
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -2175,8 +2173,8 @@ __device__ __forceinline__ long long pl_block_max(long long v, long long *red) {
 // tiles; piece c of k covers tiles [c*w/k, (c+1)*w/k).
 __device__ __forceinline__ int pl_pieces(int w, int tsplit) { return w > tsplit ? pl_div(w + tsplit - 1, tsplit) : 1; }
 
-template <int NT>
-__global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
+__global__ __launch_bounds__(PL_THREADS) void prefill_plan_kernel(AttnParams p) {
+    constexpr int NT = PL_THREADS;
     __shared__ int s_pre[PL_MAX_SEQS + 1];  // exclusive prefix of row tiles per sequence
     __shared__ int s_bk[PL_BUCKETS];        // bucket counts, then write cursors
     __shared__ int s_tmp[NT / 64];
@@ -2199,25 +2197,25 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
         if (B <= NT) s_seq[tid] = qs;
         const int v = sq < B ? pl_tiles(p, qs) : 0;
         int tot;
-        const int ex = pl_block_scan<NT>(v, s_tmp, &tot);
+        const int ex = pl_block_scan(v, s_tmp, &tot);
         if (sq < B) s_pre[sq] = carry + ex;
         carry += tot;
         int vt = v > 0 ? pl_ntk(p, qs, v - 1) : 0;
         ibig |= vt > IMG_SEQ_MAX;
         vt = min(vt, IMG_SEQ_MAX);
         int itot;
-        const int iex = pl_block_scan<NT>(vt, s_tmp, &itot);
+        const int iex = pl_block_scan(vt, s_tmp, &itot);
         if (p.pf_tbase != nullptr && sq < B) p.pf_tbase[sq] = (int)min(icarry + iex, (long long)INT32_MAX);
         icarry += itot;
     }
-    const bool img_big = pl_block_max<NT>(ibig, s_red) != 0;
+    const bool img_big = pl_block_max(ibig, s_red) != 0;
     if (tid == 0) {
         s_pre[B] = carry;
         s_nsplit = 0;
         s_nslot = 0;
         if (p.pf_tbase != nullptr) p.pf_tbase[B] = (int)min(icarry, (long long)INT32_MAX);
     }
-    pl_sync<NT>();
+    __syncthreads();
     const int n = min(carry, p.pf_items_max);
     auto seq_of = [&](int sq) { return B <= NT ? s_seq[sq] : pl_seq(p, sq); };
     // item i -> (sequence, row tile): the last sequence whose prefix is <= i
@@ -2255,8 +2253,8 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
     }
     // (the block reductions below order these stores before their reads)
     auto ntk_of = [&](int i, int sq, int rt) { return n <= NT ? s_w[i] : pl_ntk(p, seq_of(sq), rt); };
-    const long long W = pl_block_sum<NT>(wsum, s_red);
-    const long long wmax = pl_block_max<NT>(wmx, s_red);  // the longest row tile
+    const long long W = pl_block_sum(wsum, s_red);
+    const long long wmax = pl_block_max(wmx, s_red);  // the longest row tile
     long long tl = max((W * p.Hkv + p.pf_ncu - 1) / p.pf_ncu, (long long)PF_SPLIT_MIN);
     const int m = p.pf_ncu / p.Hkv;
     bool proven = false;  // the bisection's sums bound the plan: no check pass
@@ -2272,13 +2270,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
         long long hi = max(lo, (W + (cap - n) - 1) / (cap - n));
         while (lo < hi) {
             const long long mid = (lo + hi) >> 1;
-            long long P;
-            if constexpr (NT == 64) {  // 32-bit DPP sum; counts above 2^24 only need to exceed cap
-                const int k = tid < n ? pl_pieces(wt, (int)min(mid, (long long)INT32_MAX)) : 0;
-                P = __builtin_amdgcn_readfirstlane(pl_wave_sum32(min(k, 1 << 24)));
-            } else {
-                P = pl_block_sum<NT>(tid < n ? pl_pieces(wt, (int)min(mid, (long long)INT32_MAX)) : 0, s_red);
-            }
+            const long long P = pl_block_sum(tid < n ? pl_pieces(wt, (int)min(mid, (long long)INT32_MAX)) : 0, s_red);
             if (P <= cap) hi = mid;
             else lo = mid + 1;
         }
@@ -2300,16 +2292,16 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
                 ns += 1;
             }
         }
-        ex = pl_block_sum<NT>(ex, s_red);
-        sl = pl_block_sum<NT>(sl, s_red);
-        ns = pl_block_sum<NT>(ns, s_red);
+        ex = pl_block_sum(ex, s_red);
+        sl = pl_block_sum(sl, s_red);
+        ns = pl_block_sum(ns, s_red);
         if (n + ex > p.pf_grid_items || sl > p.pf_slots_max || ns > p.pf_split_max) tsplit = INT32_MAX;
     }
     // buckets that can hold an item: an unsplit row tile has at most
     // min(wmax, tsplit) key tiles, and so has a piece of a split one
     const int nb = (int)min(min(wmax, (long long)tsplit), (long long)PL_BUCKETS - 1) + 1;
     for (int b = tid; b < nb; b += NT) s_bk[b] = 0;
-    pl_sync<NT>();
+    __syncthreads();
     for (int i = tid; i < n; i += NT) {
         int sq, rt;
         locate(i, sq, rt);
@@ -2323,7 +2315,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
             atomicAdd(&s_bk[pl_bucket(q)], k - big);
         }
     }
-    pl_sync<NT>();
+    __syncthreads();
     // write cursors in descending bucket order: thread t owns the per
     // buckets nb-1-per*t .. nb-per-per*t (those >= 0)
     int total;
@@ -2334,7 +2326,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
             const int b = nb - 1 - (per * tid + k);
             if (b >= 0) loc += s_bk[b];
         }
-        int run = pl_block_scan<NT>(loc, s_tmp, &total);
+        int run = pl_block_scan(loc, s_tmp, &total);
         for (int k = 0; k < per; ++k) {
             const int b = nb - 1 - (per * tid + k);
             if (b >= 0) {
@@ -2344,7 +2336,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
             }
         }
     }
-    pl_sync<NT>();
+    __syncthreads();
     for (int i = tid; i < n; i += NT) {
         int sq, rt;
         locate(i, sq, rt);
@@ -2375,7 +2367,7 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
                                      qs.qa, {0, 0, 0}};
         }
     }
-    pl_sync<NT>();
+    __syncthreads();
     if (tid == 0) {
         p.pf_count[0] = total;
         p.pf_count[1] = s_nsplit;
@@ -2388,6 +2380,200 @@ __global__ __launch_bounds__(NT) void prefill_plan_kernel(AttnParams p) {
                          W >= (long long)PF_IMG_REUSE * icarry;
         p.pf_count[2] = fit ? 1 : 0;
         p.pf_count[3] = fit ? (int)icarry : 0;
+    }
+}
+
+// The plan of a small batch (at most 64 sequences and 64 row tiles) on one
+// wave, in registers: lane i holds sequence i, then row tile i.  The launch's
+// latency is on every short prefill's path, so nothing in it goes through a
+// loop over memory: scans and sums are DPP steps, the searches are readlane
+// loops over the sequences or row tiles there are.  (The general kernel's
+// one-wave form, with LDS scans, a bisection and a bucket sort, took 8.3 us
+// for three ragged prompts.)
+//
+// Where row tiles are few (n <= 2m, m = CUs / Hkv workgroups at a time per
+// kv-head) they are split into pieces of about t tiles that fill one round of
+// workgroups, or one more than the row tiles take, where the estimated time
+// is less, in units of a key tile: R rounds of pieces cost R (t + PW_START),
+// PW_MERGE, and PW_PART each time the split row tiles' pieces fill the device
+// (their partials go out and come back); unsplit row tiles cost the longest,
+// or with a second round the heaviest pair that heaviest-first dispatch puts
+// together.  A workgroup starts and ends in about 7 us against 1.4-2.2 us a
+// key tile (1.1 for 128-row tiles, whose partials are half as large).  With
+// more row tiles (n > 2m) a row tile longer than one CU's share of the launch
+// is cut to it, as in the general kernel.
+// Measured against the rule that cut to one CU's share, at least 16 tiles
+// (48/8 unless noted): 4 x 32 rows on 1.1-3.3K keys 53.7 -> 47 us a call,
+// 2048 contiguous keys, 8/4, 52.5 -> 42.4, 2 x 372 on 1K, 8/4, 64.6 -> 54,
+// 1252 + 242 + 1070 fresh tokens 80.2 -> 77.2 (not split; the plan itself 8.2
+// -> 7.6 us there, 7.0 -> 4.0 us with 4 row tiles).  Pieces of 4 tiles and up
+// were within 1 us of these, and 2 us worse where 5 key tiles were cut.
+#ifndef GFA_PW_START
+#define GFA_PW_START 4
+#endif
+#ifndef GFA_PW_PART
+#define GFA_PW_PART 8
+#endif
+#ifndef GFA_PW_MERGE
+#define GFA_PW_MERGE 1.5
+#endif
+#ifndef GFA_PW_SPLIT_MIN
+#define GFA_PW_SPLIT_MIN 6
+#endif
+constexpr int PW_SPLIT_MIN = GFA_PW_SPLIT_MIN;  // key tiles per piece, at least
+constexpr int PW_MAX = 64;                      // sequences, and row tiles
+constexpr int PW_PIECES = 1024;                 // pieces the kernel's table holds
+
+__global__ __launch_bounds__(64) void prefill_plan_wave_kernel(AttnParams p) {
+    __shared__ uint8_t s_map[PW_PIECES];  // work item -> row tile
+    __shared__ int s_sort[PW_MAX];
+    const int lane = threadIdx.x;
+    const int B = p.num_seqs;
+    auto rl = [](int v, int i) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(v, i); };
+    auto order = []() __attribute__((always_inline)) {  // LDS completes in order within the wave
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    // sequence `lane`
+    const int sq0 = min(lane, B - 1);
+    const PlSeq qs = pl_seq(p, sq0);
+    const int q0s = seq_q0(p, sq0);
+    const int v = lane < B ? pl_tiles(p, qs) : 0;
+    const int pre = pl_wave_scan32(v);  // inclusive
+    const int n = min(min(rl(pre, 63), p.pf_items_max), PW_MAX);
+    int icarry = 0;
+    if (p.pf_tbase != nullptr) {
+        // first image tile of each sequence (see the general kernel)
+        const int vt = v > 0 ? pl_ntk(p, qs, v - 1) : 0;
+        const bool big = pl_wave_max32(vt) > (1 << 20);
+        const int it = pl_wave_scan32(min(vt, 1 << 20));
+        if (lane < B) p.pf_tbase[lane] = it - min(vt, 1 << 20);
+        if (lane == 0) p.pf_tbase[B] = rl(it, 63);
+        icarry = big ? INT32_MAX : rl(it, 63);
+    }
+    // row tile `lane`: its sequence is the last one that starts at or before it
+    int sq = 0;
+    for (int i = 1; i < B; ++i) sq = lane >= rl(pre, i - 1) ? i : sq;
+    PlSeq q;
+    q.nq = __shfl(qs.nq, sq);
+    q.sl = __shfl(qs.sl, sq);
+    q.qa = __shfl(qs.qa, sq);
+    const int q0 = __shfl(q0s, sq);
+    const int rt = lane - __shfl(pre - v, sq);
+    const bool act = lane < n;
+    const int w = act ? pl_ntk(p, q, rt) : 0;
+    const int wmax = pl_wave_max32(w);
+    int wlo = w & 0xFFFF, whi = w >> 16;  // (the sum of 64 counts, in two halves)
+    const int64_t W = ((int64_t)pl_wave_sum32(whi) << 16) + pl_wave_sum32(wlo);
+    const int m = max(p.pf_ncu / p.Hkv, 1);
+    // place of this row tile's first piece when they are taken longest first
+    // (key: descending; ties in lane order; four row tiles a step)
+    auto place = [&](int key, int count) __attribute__((always_inline)) {
+        const int kk = key * 64 + 63 - lane;
+        int at = 0;
+        for (int i = 0; i < n; i += 4) {  // (lanes past n count 0)
+            int ki[4], ci[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ki[j] = rl(kk, i + j);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ci[j] = rl(count, i + j);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) at += ki[j] > kk ? ci[j] : 0;
+        }
+        return at;
+    };
+    int tsplit = INT32_MAX;
+    if (p.pf_slots_max > 0 && n > 0 && wmax > PW_SPLIT_MIN) {
+        if (n <= 2 * m) {
+            const bool wide = p.pf_rows == PF_ROWS;
+            int unsplit = wmax + GFA_PW_START;
+            if (n > m) {
+                const int rank = place(w, act ? 1 : 0);
+                if (act) s_sort[rank] = w;
+                order();
+                const int pair = lane < n - m ? s_sort[m - 1 - lane] + s_sort[m + lane] + 2 * GFA_PW_START : 0;
+                unsplit = max(unsplit, pl_wave_max32(pair));
+            }
+            // least t whose pieces fit the rounds, near enough: from the even
+            // share of the work, t grows by what the pieces are over
+            const int rounds = n < m ? 1 : 1 + (n + m - 1) / m;
+            const float cap = (float)(rounds * m);
+            int t = max((int)ceilf((float)W / cap), PW_SPLIT_MIN), P = INT32_MAX, k = 1;
+            for (int i = 0; i < 6 && t < wmax; ++i) {
+                k = act ? max((int)ceilf((float)w * ((1.0f - 1e-6f) / (float)t)), 1) : 0;
+                P = __builtin_amdgcn_readfirstlane(pl_wave_sum32(k));
+                if (P <= rounds * m) break;
+                t = max(t + 1, (int)((float)t * (float)P / cap));
+            }
+            if (t < wmax && P <= min(rounds * m, p.pf_slots_max)) {
+                const int S = __builtin_amdgcn_readfirstlane(pl_wave_sum32(k > 1 ? k : 0));
+                const float cost = (float)(rounds * (t + GFA_PW_START)) + (wide ? 1.0f : 2.0f) * GFA_PW_MERGE +
+                                   (wide ? 1.0f : 0.5f) * GFA_PW_PART * (float)S / (float)m;
+                if (cost < (float)unsplit) tsplit = t;
+            }
+        } else {
+            const int64_t share = max((W * p.Hkv + p.pf_ncu - 1) / p.pf_ncu, (int64_t)PF_SPLIT_MIN);
+            if (share < wmax) tsplit = (int)share;
+        }
+    }
+    int k = act ? pl_pieces(w, tsplit) : 0;
+    int total = pl_wave_sum32(k);
+    int ssum = pl_wave_scan32(k > 1 ? k : 0);
+    uint64_t smask = __ballot(k > 1);
+    if (total > min(p.pf_grid_items, PW_PIECES) || rl(ssum, 63) > p.pf_slots_max ||
+        __builtin_popcountll(smask) > p.pf_split_max) {  // past the workspace: nothing is cut
+        k = act ? 1 : 0;
+        total = n;
+        ssum = 0;
+        smask = 0;
+    }
+    const int slot0 = ssum - k;
+    if (k > 1) {
+        int *e = p.pf_split + 4 * __builtin_popcountll(smask & (((uint64_t)1 << lane) - 1));
+        e[0] = sq;
+        e[1] = rt;
+        e[2] = slot0;
+        e[3] = k;
+    }
+    // heaviest first, by the row tile's piece size (a row tile's pieces follow
+    // each other); in any order where all run at once
+    const int at = total > m ? place(k > 0 ? pl_div(w + k - 1, k) : -1, k) : pl_wave_scan32(k) - k;
+    if (pl_wave_max32(k) <= 16) {
+        for (int c = 0; c < k; ++c) s_map[at + c] = (uint8_t)lane;
+    } else {
+        for (int i = 0; i < n; ++i)
+            for (int c = lane; c < rl(k, i); c += 64) s_map[rl(at, i) + c] = (uint8_t)i;
+    }
+    order();
+    for (int base = 0; base < total; base += 64) {
+        const int x = base + lane;
+        const int i = s_map[min(x, total - 1)];
+        const int wi = __shfl(w, i), ki = __shfl(k, i), c = x - __shfl(at, i), sl0 = __shfl(slot0, i);
+        PfItem it;
+        it.s = __shfl(sq, i);
+        it.rt = __shfl(rt, i);
+        it.q0 = __shfl(q0, i);
+        it.nq = __shfl(q.nq, i);
+        it.sl = __shfl(q.sl, i);
+        it.qa = __shfl(q.qa, i);
+        it.pad[0] = it.pad[1] = it.pad[2] = 0;
+        if (x >= total) continue;
+        // piece c of ki: tiles [c wi / ki, (c + 1) wi / ki), the remainder of
+        // wi / ki spread over the pieces
+        const int qd = pl_div(wi, ki), rw = wi - qd * ki;
+        it.kt0 = ki > 1 ? c * qd + pl_div(c * rw, ki) : 0;
+        it.kt1 = ki > 1 ? (c + 1) * qd + pl_div((c + 1) * rw, ki) : INT32_MAX;
+        it.slot = ki > 1 ? sl0 + c : -1;
+        p.pf_items[x] = it;
+    }
+    if (lane == 0) {
+        p.pf_count[0] = total;
+        p.pf_count[1] = __builtin_popcountll(smask);
+        // the tile images: all of them or none (see the general kernel)
+        const bool fit = p.pf_tiles != nullptr && icarry != INT32_MAX &&
+                         icarry <= p.pf_tiles_cap / ((int64_t)p.Hkv * PF_IMG_BYTES) && W >= (int64_t)PF_IMG_REUSE * icarry;
+        p.pf_count[2] = fit ? 1 : 0;
+        p.pf_count[3] = fit ? icarry : 0;
     }
 }
 
@@ -3158,11 +3344,8 @@ Plan bound_plan(int max_num_seqs, int64_t max_num_tokens, int num_heads, int num
 
 // The plan kernel of a prefill launch with a work list.
 void launch_plan(const AttnParams &p, const Plan &pl, int num_seqs, hipStream_t stream) {
-    // one wave for small batches: its scans and reductions need no
-    // barriers across 16 waves (8 x (32768 + 12) at 48/8: 18.6 us with
-    // 1024 threads)
-    if (num_seqs <= 64 && pl.pf_items_max <= 64) prefill_plan_kernel<64><<<1, 64, 0, stream>>>(p);
-    else prefill_plan_kernel<PL_THREADS><<<1, PL_THREADS, 0, stream>>>(p);
+    if (num_seqs <= PW_MAX && pl.pf_items_max <= PW_MAX) prefill_plan_wave_kernel<<<1, 64, 0, stream>>>(p);
+    else prefill_plan_kernel<<<1, PL_THREADS, 0, stream>>>(p);
 }
 
 // The workspace's prefill regions (no tile images).
@@ -3682,8 +3865,8 @@ Plan flat_plan(int batch, int seq_q, int num_heads, int num_kv_heads, int seq_kv
     pl.ndc = 0;
     pl.need_prefill = true;
     pl.pf_rows = PF_ROWS;
-    plan_finish(pl, batch, (int64_t)batch * seq_q, num_heads / num_kv_heads, num_kv_heads, false, nkt > PF_SPLIT_MIN,
-                seq_kv, 0, (nkt + PF_SPLIT_MIN - 1) / PF_SPLIT_MIN);
+    plan_finish(pl, batch, (int64_t)batch * seq_q, num_heads / num_kv_heads, num_kv_heads, false, nkt > PW_SPLIT_MIN,
+                seq_kv, 0, (nkt + PW_SPLIT_MIN - 1) / PW_SPLIT_MIN);
     pl.img_bytes = (size_t)batch * nkt * num_kv_heads * PF_IMG_BYTES;
     return pl;
 }
