@@ -196,6 +196,10 @@ __device__ __forceinline__ void store_out(void *out, int64_t off, float v) {
 template <int ODT>
 __device__ __forceinline__ uint32_t pack2_out(float a, float b) {
     if constexpr (ODT == GFA_DTYPE_F16) {
+        // the fp32 values first (an fp16 output is the fp32 one rounded): no
+        // multiply may be folded into the conversion (v_fma_mix)
+        asm("" : "+v"(a));
+        asm("" : "+v"(b));
         return (uint32_t)__builtin_bit_cast(uint16_t, (half_t)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (half_t)b) << 16);
     } else {
         const uint32_t u = __float_as_uint(a), v = __float_as_uint(b);
