@@ -698,8 +698,8 @@ struct SegInfo {
 // the sequence belongs to the prefill kernel.
 __device__ __forceinline__ SegInfo seg_info(const AttnParams &p, int s) {
     SegInfo si;
-    si.q0 = p.qsl[s];
-    si.nq = p.qsl[s + 1] - si.q0;
+    si.q0 = seq_q0(p, s);
+    si.nq = seq_nq(p, s);
     si.sl = p.seq_lens[s];
     si.qa = p.q_abs ? p.q_abs[s] : si.sl - si.nq;
     si.kv_lim = p.causal ? min(si.sl, max(si.qa + si.nq, 0)) : si.sl;
@@ -2615,7 +2615,7 @@ __global__ __launch_bounds__(64 * PF_NSP) void prefill_tiles_kernel(AttnParams p
         }
         const int s = __builtin_amdgcn_readfirstlane(lo);
         const int kt = tix - p.pf_tbase[s];
-        const int nq = p.qsl[s + 1] - p.qsl[s];
+        const int nq = seq_nq(p, s);
         const int sl = p.seq_lens[s];
         const int qa = p.q_abs ? p.q_abs[s] : sl - nq;
         const int kv_lim = p.causal ? min(sl, max(qa + nq, 0)) : sl;
@@ -3324,6 +3324,22 @@ Plan make_plan(int num_seqs, int num_tokens, int num_heads, int num_kv_heads, in
     return pl;
 }
 
+// Masks whose rows start 8-byte aligned and hold whole runs of 4 keys: a
+// lane's four adjacent keys come in one load.
+int mask_vec(const void *mask, int64_t batch_stride, int64_t row_stride, int cols) {
+    return mask != nullptr && ((uintptr_t)mask & 7) == 0 && (batch_stride & 3) == 0 && (row_stride & 3) == 0 &&
+           (cols & 3) == 0;
+}
+
+// A masked batch: every sequence through the prefill kernel, in 256-row tiles.
+Plan make_masked_plan(int num_seqs, int num_tokens, int num_heads, int num_kv_heads) {
+    Plan pl{};
+    pl.need_prefill = true;
+    pl.pf_rows = PF_ROWS;
+    plan_finish(pl, num_seqs, num_tokens, num_heads / num_kv_heads, num_kv_heads, false, true, 0, 0);
+    return pl;
+}
+
 // A plan whose every workspace region is at least that of any make_plan()
 // call with num_seqs <= max_num_seqs and num_tokens <= max_num_tokens (any
 // max_query_len, any mix of decode and prefill sequences): each decode class
@@ -3426,9 +3442,13 @@ hipError_t launch_all(const AttnParams &p0, const Plan &pl, char *ws, int num_se
         const int rows = max_query_len * p.G;
         const int tiles = (rows + pl.pf_rows - 1) / pl.pf_rows;
         const dim3 grid = p.pf_items ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, num_seqs);
-        if (pl.pf_rows == PF_ROWS) attn_prefill_kernel<QDT, ODT, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+        if (p.mask) {  // (padded batches: fp32 output, 256-row tiles)
+            if constexpr (ODT == GFA_DTYPE_F32)
+                attn_prefill_kernel<QDT, ODT, false, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+        } else if (pl.pf_rows == PF_ROWS)
+            attn_prefill_kernel<QDT, ODT, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
         else attn_prefill_kernel<QDT, ODT, false, false, 2><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
-        if (p.pf_items && pl.pf_split_max)  // returns at once when the plan split nothing
+        if (p.pf_items && pl.pf_slots_max)  // returns at once when the plan split nothing
             attn_prefill_combine_kernel<ODT><<<device_cus() * GFA_PFC_WGS_PER_CU, 256, 0, stream>>>(p);
     }
     return hipGetLastError();
@@ -3542,6 +3562,15 @@ extern "C" hipError_t gfx906_fa_amd_noalloc_scratch_copy(void *dst, size_t offse
 
 namespace {
 
+// A padded batch: q [num_seqs, heads, uq, 128] and out alike (token stride 128,
+// query_start_loc absent), and its optional additive mask.
+struct Padded {
+    int uq;
+    const void *mask;
+    int64_t mask_bs, mask_rs;
+    int mask_cols;
+};
+
 // The step's new K/V rows for the fused cache write (element strides).
 struct NewKV {
     const void *key, *value;
@@ -3558,7 +3587,7 @@ hipError_t paged_attention_impl(
     int causal, int num_seqs, int num_tokens, int num_heads, int num_kv_heads, int head_size,
     int block_size, int max_query_len, int max_seq_len, float scale, void *out, int out_dtype,
     int64_t out_token_stride, int64_t out_head_stride, void *workspace, size_t workspace_bytes,
-    const NewKV *nkv, hipStream_t stream, bool noalloc = false) {
+    const NewKV *nkv, hipStream_t stream, bool noalloc = false, const Padded *padded = nullptr) {
     if (nkv && num_tokens > 0) {
         const uint64_t align = nkv->dtype == GFA_DTYPE_F32 ? 8 : 4;  // two values per lane
         if (nkv->dtype != q_dtype ||
@@ -3595,7 +3624,9 @@ hipError_t paged_attention_impl(
         return hipErrorInvalidValue;
     }
     const int G = num_heads / num_kv_heads;
-    Plan pl = make_plan(num_seqs, num_tokens, num_heads, num_kv_heads, max(max_query_len, 1), max(max_seq_len, 1));
+    const bool masked = padded && padded->mask;
+    Plan pl = masked ? make_masked_plan(num_seqs, num_tokens, num_heads, num_kv_heads)
+                     : make_plan(num_seqs, num_tokens, num_heads, num_kv_heads, max(max_query_len, 1), max(max_seq_len, 1));
     if (noalloc) {
         // the library's scratch array instead of a caller workspace; a plan
         // whose split-prefill partials do not fit leaves row tiles unsplit
@@ -3639,8 +3670,14 @@ hipError_t paged_attention_impl(
     p.bt_stride = block_table_stride;
     p.seq_lens = seq_lens;
     p.qsl = query_start_loc;
-    p.uq = p.uq_rows = 0;
+    p.uq = padded ? padded->uq : 0;
+    p.uq_rows = padded ? num_heads * padded->uq : 0;
     p.kv_cap = INT32_MAX;
+    p.mask = masked ? static_cast<const uint16_t *>(padded->mask) : nullptr;
+    p.mask_bs = masked ? padded->mask_bs : 0;
+    p.mask_rs = masked ? padded->mask_rs : 0;
+    p.mask_cols = masked ? padded->mask_cols : 0;
+    p.mask_vec = masked ? mask_vec(padded->mask, padded->mask_bs, padded->mask_rs, padded->mask_cols) : 0;
     p.q_abs = q_abs_offset;
     p.causal = causal ? 1 : 0;
     p.Hkv = num_kv_heads;
@@ -3745,6 +3782,33 @@ extern "C" hipError_t gfx906_fa_amd_paged_attention_noalloc(
                                 nullptr, stream, true);
 }
 
+extern "C" size_t gfx906_fa_amd_paged_attention_padded_workspace_size(int batch, int seq_q, int num_heads,
+                                                                     int num_kv_heads, int max_seq_len, int masked) {
+    if (batch <= 0 || seq_q <= 0 || num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads) return 256;
+    return masked ? make_masked_plan(batch, batch * seq_q, num_heads, num_kv_heads).bytes
+                  : gfx906_fa_amd_paged_attention_workspace_size(batch, batch * seq_q, num_heads, num_kv_heads, 128,
+                                                                 seq_q, max_seq_len);
+}
+
+extern "C" hipError_t gfx906_fa_amd_paged_attention_padded(
+    const void *q, int q_dtype, const uint8_t *k_cache, const uint8_t *v_cache, int64_t cache_block_stride,
+    int64_t cache_head_stride, const int32_t *block_table, int64_t block_table_stride, const int32_t *seq_lens,
+    const int32_t *q_abs_offset, const void *mask, int64_t mask_batch_stride, int64_t mask_row_stride, int mask_cols,
+    int batch, int seq_q, int num_heads, int num_kv_heads, int head_size, int block_size, int max_seq_len, float scale,
+    float *out, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (mask && (q_abs_offset || mask_cols < 0)) {
+        fprintf(stderr, "[gfx906_fa_amd] paged_attention_padded: mask excludes q_abs_offset\n");
+        return hipErrorInvalidValue;
+    }
+    const Padded pd{seq_q, mask, mask_batch_stride, mask_row_stride, mask_cols};
+    const int64_t hs = (int64_t)seq_q * 128;
+    return paged_attention_impl(q, q_dtype, 128, hs, k_cache, v_cache, cache_block_stride, cache_head_stride,
+                                block_table, block_table_stride, seq_lens, nullptr, q_abs_offset,
+                                q_abs_offset != nullptr, batch, batch * seq_q, num_heads, num_kv_heads, head_size,
+                                block_size, seq_q, max_seq_len, scale, out, GFA_DTYPE_F32, 128, hs, workspace,
+                                workspace_bytes, nullptr, stream, false, &pd);
+}
+
 extern "C" hipError_t gfx906_fa_amd_paged_attention_kv_write(
     const void *q, int q_dtype, int64_t q_token_stride, int64_t q_head_stride,
     const uint8_t *k_cache, const uint8_t *v_cache, int64_t cache_block_stride,
@@ -3771,13 +3835,6 @@ extern "C" hipError_t gfx906_fa_amd_paged_attention_kv_write(
 }
 
 namespace {
-
-// Masks whose rows start 8-byte aligned and hold whole runs of 4 keys: a
-// lane's four adjacent keys come in one load.
-int mask_vec(const void *mask, int64_t batch_stride, int64_t row_stride, int cols) {
-    return mask != nullptr && ((uintptr_t)mask & 7) == 0 && (batch_stride & 3) == 0 && (row_stride & 3) == 0 &&
-           (cols & 3) == 0;
-}
 
 // Pieces per segment of the contiguous decode: enough single-wave
 // workgroups to fill the device (8 per CU), each at least FD_MIN_SUB

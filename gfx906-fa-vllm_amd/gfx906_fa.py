@@ -93,6 +93,9 @@ def _load():
         "gfx906_fa_amd_flat_decode_workspace_size": (SZ, [I, I, I, I, I]),
         "gfx906_fa_amd_flat_decode": (I, [P, I, I64, I64, P, P, P, P, I, I, I, I, I, I, F, P, I64, I64,
                                           P, SZ, P]),
+        "gfx906_fa_amd_paged_attention_padded_workspace_size": (SZ, [I, I, I, I, I, I]),
+        "gfx906_fa_amd_paged_attention_padded": (I, [P, I, P, P, I64, I64, P, I64, P, P, P, I64, I64, I,
+                                                     I, I, I, I, I, I, I, F, P, P, SZ, P]),
         "gfx906_fa_amd_flat_attention_workspace_size": (SZ, [I, I, I, I, I, I]),
         "gfx906_fa_amd_flat_attention": (I, [P, P, P, P, P, P, I64, I64, I, I, I, I, I, I, I, F, P, P, SZ, P]),
         "gfx906_fa_amd_paged_attention_tiled": (I, [P, I, I64, I64, P, P, I, I64, I64, I64, I64, P, I64,
@@ -641,32 +644,33 @@ def forward_paged_direct(q: torch.Tensor, key_cache_q8: torch.Tensor, value_cach
     B, Hq, Sq, D = q.shape
     _check(block_table.shape[0] == B, "block_table[0] must equal batch")
     _check(seq_lens.dim() == 1 and seq_lens.shape[0] == B, "seq_lens must be [batch]")
-    q_bshd = q.transpose(1, 2).reshape(B * Sq, Hq, D)
-    qsl = torch.arange(0, (B + 1) * Sq, Sq, dtype=torch.int32, device=q.device)
-    bt = block_table if block_table.dtype == torch.int32 else block_table.to(torch.int32)
-    sl = seq_lens if seq_lens.dtype == torch.int32 else seq_lens.to(torch.int32)
+    bt = (block_table if block_table.dtype == torch.int32 else block_table.to(torch.int32)).contiguous()
+    sl = (seq_lens if seq_lens.dtype == torch.int32 else seq_lens.to(torch.int32)).contiguous()
     max_kv = bt.shape[1] * (key_cache_q8.shape[2] // SUBPAGE_BYTES * SUBPAGE_TOKENS)
-    if mask is None:
-        out = paged_attention(q_bshd, key_cache_q8, value_cache, bt.contiguous(), sl.contiguous(), qsl,
-                              Sq, max_kv, scale, q_abs_offset=q_abs_offset,
-                              causal=q_abs_offset is not None, out_dtype=torch.float32)
-        return out.view(B, Sq, Hq, D).transpose(1, 2).contiguous()
-    # materialised mask: the tiled kernel over the same planar Q8 planes
     mk, mbs, mrs, mcols = _mask_args(mask, B, Sq, q_abs_offset)
-    q_bshd = q_bshd.contiguous()
-    sl = sl.contiguous()
-    _check(q_bshd.dtype in _DT, "q must be fp32, fp16 or bf16")
+    _cuda(bt, "block_table")
+    _cuda(sl, "seq_lens")
+    _check(q.dtype in _DT, "query must be fp16, bf16 or fp32")
+    _check(D == 128, "query must be [B, Hq, Sq, 128]")
+    out = torch.empty((B, Hq, Sq, D), dtype=torch.float32, device=q.device)
+    if B * Sq == 0:  # no query rows
+        return out
     bs, Hkv, cbs, chs = _plane_info(key_cache_q8, value_cache)
     _check(Hq % Hkv == 0, f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
-    out = torch.empty((B * Sq, Hq, D), dtype=torch.float32, device=q.device)
-    bt = bt.contiguous()
-    err = _load().gfx906_fa_amd_paged_attention_tiled(
-        _ptr(q_bshd), _DT[q_bshd.dtype], q_bshd.stride(0), q_bshd.stride(1), _ptr(key_cache_q8),
-        _ptr(value_cache), 0, cbs, chs, cbs, chs, _ptr(bt), bt.stride(0), _ptr(sl),
-        _ptr(qsl), None, 0, _ptr(mk), mbs, mrs, mcols, B, B * Sq, Hq, Hkv, D, bs, Sq, float(scale),
-        _ptr(out), out.stride(0), out.stride(1), _stream(q.device))
-    _ok(err, "gfx906_fa_amd_paged_attention_tiled")
-    return out.view(B, Sq, Hq, D).transpose(1, 2).contiguous()
+    _check(bt.dim() == 2, "block_table must be int32 [num_seqs, max_blocks] with contiguous rows")
+    if q_abs_offset is not None:
+        _cuda(q_abs_offset, "q_abs_offset")
+        _check(q_abs_offset.dtype == torch.int32 and q_abs_offset.is_contiguous()
+               and q_abs_offset.shape[0] >= B, "q_abs_offset must be int32 [B]")
+    qc = q.contiguous()
+    L = _load()
+    ws = new_workspace(L.gfx906_fa_amd_paged_attention_padded_workspace_size(B, Sq, Hq, Hkv, max_kv, mk is not None),
+                       q.device)
+    _ok(L.gfx906_fa_amd_paged_attention_padded(
+        _ptr(qc), _DT[qc.dtype], _ptr(key_cache_q8), _ptr(value_cache), cbs, chs, _ptr(bt), bt.stride(0), _ptr(sl),
+        _ptr(q_abs_offset), _ptr(mk), mbs, mrs, mcols, B, Sq, Hq, Hkv, D, bs, max_kv, float(scale), _ptr(out), _ptr(ws),
+        ws.numel(), _stream(q.device)), "gfx906_fa_amd_paged_attention_padded")
+    return out
 
 
 # ---------------------------------------------------------------------------

@@ -428,6 +428,24 @@ hipError_t gfx906_fa_amd_flat_attention(
     int num_heads, int num_kv_heads, int seq_kv, int head_size, float scale, float *out, void *workspace,
     size_t workspace_bytes, hipStream_t stream);
 
+/* (9) Padded-batch paged attention (gfx906_fa_launch_paged's own batch layout,
+ *     extension/gfx906_fa.cpp:516-658): q [batch][num_heads][seq_q][128]
+ *     (q_dtype) and out fp32 alike, both contiguous, over the planar cache as
+ *     (5).  Without q_abs_offset every row sees all seq_lens[b] keys; with
+ *     it, row j sees keys k <= q_abs_offset[b] + j.  mask as in (7), exclusive
+ *     with q_abs_offset; masked batches run the tiled kernel, split over the
+ *     keys as (5)'s prefill is.  workspace:
+ *     gfx906_fa_amd_paged_attention_padded_workspace_size() bytes, 256-byte
+ *     aligned, no initial contents. */
+size_t gfx906_fa_amd_paged_attention_padded_workspace_size(int batch, int seq_q, int num_heads, int num_kv_heads,
+                                                           int max_seq_len, int masked);
+hipError_t gfx906_fa_amd_paged_attention_padded(
+    const void *q, int q_dtype, const uint8_t *k_cache, const uint8_t *v_cache, int64_t cache_block_stride,
+    int64_t cache_head_stride, const int32_t *block_table, int64_t block_table_stride, const int32_t *seq_lens,
+    const int32_t *q_abs_offset, const void *mask, int64_t mask_batch_stride, int64_t mask_row_stride, int mask_cols,
+    int batch, int seq_q, int num_heads, int num_kv_heads, int head_size, int block_size, int max_seq_len, float scale,
+    float *out, void *workspace, size_t workspace_bytes, hipStream_t stream);
+
 /* Measurement helper: streams `bytes` (a multiple of 16) from the 16-byte
  * aligned device buffer `src` with non-temporal 16-byte loads and writes one
  * XOR word per wave to `out` (at least gfx906_fa_amd_stream_read_words()
