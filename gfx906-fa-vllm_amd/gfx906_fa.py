@@ -127,12 +127,26 @@ def _cuda(t: torch.Tensor, name: str) -> None:
     _check(t.is_cuda, f"{name} must be CUDA/HIP")
 
 
+# The calls below are launch-bound at small sizes (a 3-sequence decode step took
+# 33 us of host time for 19 us of device work), so their checks are plain
+# conditions: messages are formatted only on failure, pointers go to ctypes as
+# integers, and the raw stream handle is read without building a Stream.
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    if _raw_stream is None or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
+
+
+def _all_cuda(tensors, names: str) -> None:
+    for t, n in zip(tensors, names.split()):
+        _cuda(t, n)
 
 
 def _ok(err: int, what: str) -> None:
@@ -217,14 +231,15 @@ def gather_paged_kv_q8(key_cache_q8: torch.Tensor, value_cache: torch.Tensor,
     _check(value_cache.shape[1] == bs, "value_cache block_size mismatch")
     _check(value_cache.shape[2] == Hkv, "value_cache Hkv mismatch")
     _check(D % QK8_0 == 0, "D must be multiple of 32")
-    _check(bpr == D // QK8_0 * Q8_0_BYTES,
-           f"bytes_per_row must equal (D/32)*34, got {bpr} vs expected {D // QK8_0 * Q8_0_BYTES}")
+    if bpr != D // QK8_0 * Q8_0_BYTES:
+        raise RuntimeError(f"bytes_per_row must equal (D/32)*34, got {bpr} vs expected {D // QK8_0 * Q8_0_BYTES}")
     _check(block_table.dtype == torch.int32, "block_table must be int32 (caller should .to(torch.int32))")
     _check(block_table.is_contiguous(), "block_table must be contiguous")
     _check(seq_lens.is_contiguous(), "seq_lens must be contiguous")
     B, M = block_table.shape
     _check(seq_lens.shape[0] == B, "seq_lens vs block_table batch mismatch")
-    _check(Sk > 0 and Sk % 32 == 0, f"Sk must be positive multiple of 32, got {Sk}")
+    if Sk <= 0 or Sk % 32:
+        raise RuntimeError(f"Sk must be positive multiple of 32, got {Sk}")
     _check(key_cache_q8.stride(3) == 1 and value_cache.stride(3) == 1, "cache rows must be contiguous")
     vrow = value_cache.shape[3]
 
@@ -264,40 +279,54 @@ def _plane_info(key_cache: torch.Tensor, value_cache: torch.Tensor):
     """Validates a planar (K, V) plane pair [NB, Hkv, bs/16*2176] (uint8, any
     block/head strides, contiguous pages) -> (block_size, Hkv, block stride,
     head stride)."""
-    _check(key_cache.dtype == torch.uint8 and value_cache.dtype == torch.uint8,
-           "key_cache / value_cache must be uint8 planar Q8 planes")
-    _check(key_cache.dim() == 3 and value_cache.dim() == 3,
-           "key_cache / value_cache must be [num_blocks, Hkv, block_size/16*2176]")
-    _check(key_cache.shape == value_cache.shape, "key_cache / value_cache shape mismatch")
-    _check(key_cache.stride() == value_cache.stride(), "key_cache / value_cache stride mismatch")
-    NB, Hkv, nbytes = key_cache.shape
-    _check(nbytes % SUBPAGE_BYTES == 0, "page bytes must be a multiple of 2176")
-    _check(key_cache.stride(2) == 1, "pages must be contiguous")
-    return nbytes // SUBPAGE_BYTES * SUBPAGE_TOKENS, Hkv, key_cache.stride(0), key_cache.stride(1)
+    if key_cache.dtype != torch.uint8 or value_cache.dtype != torch.uint8:
+        raise RuntimeError("key_cache / value_cache must be uint8 planar Q8 planes")
+    shape, strides = key_cache.shape, key_cache.stride()
+    if len(shape) != 3 or value_cache.dim() != 3:
+        raise RuntimeError("key_cache / value_cache must be [num_blocks, Hkv, block_size/16*2176]")
+    if shape != value_cache.shape:
+        raise RuntimeError("key_cache / value_cache shape mismatch")
+    if strides != value_cache.stride():
+        raise RuntimeError("key_cache / value_cache stride mismatch")
+    subs, rest = divmod(shape[2], SUBPAGE_BYTES)
+    if rest:
+        raise RuntimeError("page bytes must be a multiple of 2176")
+    if strides[2] != 1:
+        raise RuntimeError("pages must be contiguous")
+    return subs * SUBPAGE_TOKENS, shape[1], strides[0], strides[1]
 
 
 def reshape_and_cache_q8_kv(key: torch.Tensor, value: torch.Tensor, slot_mapping: torch.Tensor,
                             key_cache: torch.Tensor, value_cache: torch.Tensor) -> None:
     """Quantize key and value [T, Hkv, 128] to Q8_0 and write them at
     slot_mapping into the planar planes (one launch; slot < 0 skips)."""
-    for t, n in ((key, "key"), (value, "value"), (slot_mapping, "slot_mapping"),
-                 (key_cache, "key_cache"), (value_cache, "value_cache")):
-        _cuda(t, n)
-    _check(key.dtype in _DT and value.dtype == key.dtype, "key/value must share dtype fp16/bf16/fp32")
-    _check(key.dim() == 3 and value.shape == key.shape, "key/value must be [num_tokens, Hkv, D]")
-    _check(slot_mapping.dtype == torch.int64, "slot_mapping must be int64")
+    if not (key.is_cuda and value.is_cuda and slot_mapping.is_cuda and key_cache.is_cuda and value_cache.is_cuda):
+        _all_cuda((key, value, slot_mapping, key_cache, value_cache), "key value slot_mapping key_cache value_cache")
+    dt = _DT.get(key.dtype)
+    if dt is None or value.dtype != key.dtype:
+        raise RuntimeError("key/value must share dtype fp16/bf16/fp32")
+    if key.dim() != 3 or value.shape != key.shape:
+        raise RuntimeError("key/value must be [num_tokens, Hkv, D]")
+    if slot_mapping.dtype != torch.int64:
+        raise RuntimeError("slot_mapping must be int64")
     T, Hkv, D = key.shape
-    _check(D == 128, "head_size must be 128")
-    _check(key.stride(2) == 1 and value.stride(2) == 1, "key/value rows must be contiguous")
-    _check(slot_mapping.shape[0] == T, "slot_mapping length mismatch")
+    if D != 128:
+        raise RuntimeError("head_size must be 128")
+    kts, khs, ks = key.stride()
+    vts, vhs, vs = value.stride()
+    if ks != 1 or vs != 1:
+        raise RuntimeError("key/value rows must be contiguous")
+    if slot_mapping.shape[0] != T:
+        raise RuntimeError("slot_mapping length mismatch")
     bs, Hc, cbs, chs = _plane_info(key_cache, value_cache)
-    _check(Hc == Hkv, f"cache Hkv mismatch: got {Hc} vs key Hkv={Hkv}")
+    if Hc != Hkv:
+        raise RuntimeError(f"cache Hkv mismatch: got {Hc} vs key Hkv={Hkv}")
     sm = slot_mapping.contiguous()
     err = _load().gfx906_fa_amd_cache_write_kv(
-        _ptr(key), _ptr(value), _DT[key.dtype], _ptr(sm), _ptr(key_cache), _ptr(value_cache), T,
-        Hkv, D, bs, key.stride(0), key.stride(1), value.stride(0), value.stride(1), cbs, chs,
-        _stream(key.device))
-    _ok(err, "gfx906_fa_amd_cache_write_kv")
+        key.data_ptr(), value.data_ptr(), dt, sm.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), T, Hkv, D,
+        bs, kts, khs, vts, vhs, cbs, chs, _stream(key.device))
+    if err:
+        _ok(err, "gfx906_fa_amd_cache_write_kv")
 
 
 def rope_and_cache_q8_kv(positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor,
@@ -310,10 +339,10 @@ def rope_and_cache_q8_kv(positions: torch.Tensor, query: torch.Tensor, key: torc
     pairs; per-operation rounding in the model dtype), then the rotated key
     and the value quantized to Q8_0 at slot_mapping (< 0 skips) - one launch.
     Positions outside [0, max_position) leave their rows unrotated."""
-    for t, n in ((positions, "positions"), (query, "query"), (key, "key"), (value, "value"),
-                 (cos_sin_cache, "cos_sin_cache"), (slot_mapping, "slot_mapping"),
-                 (key_cache, "key_cache"), (value_cache, "value_cache")):
-        _cuda(t, n)
+    if not (positions.is_cuda and query.is_cuda and key.is_cuda and value.is_cuda and cos_sin_cache.is_cuda
+            and slot_mapping.is_cuda and key_cache.is_cuda and value_cache.is_cuda):
+        _all_cuda((positions, query, key, value, cos_sin_cache, slot_mapping, key_cache, value_cache),
+                  "positions query key value cos_sin_cache slot_mapping key_cache value_cache")
     _check(query.dtype in (torch.float16, torch.bfloat16) and key.dtype == query.dtype
            and value.dtype == query.dtype, "query/key/value must share dtype fp16 or bf16")
     _check(query.dim() == 3 and key.dim() == 3 and value.shape == key.shape and query.shape[0] == key.shape[0],
@@ -327,12 +356,14 @@ def rope_and_cache_q8_kv(positions: torch.Tensor, query: torch.Tensor, key: torc
     T, Hq, D = query.shape
     Hkv = key.shape[1]
     _check(D == 128 and key.shape[2] == 128, "head_size must be 128")
-    for t, n in ((query, "query"), (key, "key"), (value, "value")):
-        _check(t.stride(2) == 1, f"{n} rows must be contiguous")
+    if query.stride(2) != 1 or key.stride(2) != 1 or value.stride(2) != 1:
+        raise RuntimeError("query, key and value rows must be contiguous")
     rot = cos_sin_cache.shape[1] if rot_dim is None else int(rot_dim)
     bs, Hc, cbs, chs = _plane_info(key_cache, value_cache)
-    _check(Hc == Hkv, f"cache Hkv mismatch: got {Hc} vs key Hkv={Hkv}")
-    _check(Hq % Hkv == 0, f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
+    if Hc != Hkv:
+        raise RuntimeError(f"cache Hkv mismatch: got {Hc} vs key Hkv={Hkv}")
+    if Hq % Hkv:
+        raise RuntimeError(f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
     pos = positions.contiguous()
     sm = slot_mapping.contiguous()
     err = _load().gfx906_fa_amd_rope_cache_write_kv(
@@ -360,7 +391,8 @@ def gather_paged_kv_q8q8(key_cache: torch.Tensor, value_cache: torch.Tensor,
     bs, Hkv, cbs, chs = _plane_info(key_cache, value_cache)
     B, M = block_table.shape
     _check(seq_lens.shape[0] == B, "seq_lens vs block_table batch mismatch")
-    _check(Sk > 0 and Sk % 32 == 0, f"Sk must be positive multiple of 32, got {Sk}")
+    if Sk <= 0 or Sk % 32:
+        raise RuntimeError(f"Sk must be positive multiple of 32, got {Sk}")
 
     def use_or_alloc(buf):
         if (buf is not None and tuple(buf.shape) == (B, Hkv, Sk, 136) and buf.dtype == torch.uint8
@@ -476,46 +508,58 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
     ``slot_mapping`` (int64 [T]) the step's K/V are first written to the cache
     as ``reshape_and_cache_q8_kv`` does; decode-shaped batches do it inside
     the attention launch."""
-    for t, n in ((query, "query"), (block_table, "block_table"), (seq_lens, "seq_lens"),
-                 (query_start_loc, "query_start_loc")):
-        _cuda(t, n)
-    _check(query.dtype in _DT, "query must be fp16, bf16 or fp32")
-    _check(query.dim() == 3 and query.shape[2] == 128, "query must be [num_tokens, Hq, 128]")
+    if not (query.is_cuda and block_table.is_cuda and seq_lens.is_cuda and query_start_loc.is_cuda):
+        _all_cuda((query, block_table, seq_lens, query_start_loc), "query block_table seq_lens query_start_loc")
+    dev = query.device
+    qdt = _DT.get(query.dtype)
+    if qdt is None:
+        raise RuntimeError("query must be fp16, bf16 or fp32")
+    if query.dim() != 3 or query.shape[2] != 128:
+        raise RuntimeError("query must be [num_tokens, Hq, 128]")
     T, Hq, D = query.shape
     if T == 0:  # no query rows: nothing to compute or write (an empty tensor's strides are arbitrary)
-        return out if out is not None else torch.empty((0, Hq, D), dtype=out_dtype or query.dtype,
-                                                       device=query.device)
-    _check(query.stride(2) == 1, "query rows must be contiguous")
+        return out if out is not None else torch.empty((0, Hq, D), dtype=out_dtype or query.dtype, device=dev)
+    qts, qhs, qs = query.stride()
+    if qs != 1:
+        raise RuntimeError("query rows must be contiguous")
     bs, Hkv, cbs, chs = _plane_info(key_cache, value_cache)
-    _check(Hq % Hkv == 0, f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
-    _check(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1,
-           "block_table must be int32 [num_seqs, max_blocks] with contiguous rows")
-    _check(seq_lens.dtype == torch.int32 and seq_lens.is_contiguous(), "seq_lens must be contiguous int32")
-    _check(query_start_loc.dtype == torch.int32 and query_start_loc.is_contiguous(),
-           "query_start_loc must be contiguous int32")
+    if Hq % Hkv:
+        raise RuntimeError(f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
+    if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1:
+        raise RuntimeError("block_table must be int32 [num_seqs, max_blocks] with contiguous rows")
+    if seq_lens.dtype != torch.int32 or not seq_lens.is_contiguous():
+        raise RuntimeError("seq_lens must be contiguous int32")
+    if query_start_loc.dtype != torch.int32 or not query_start_loc.is_contiguous():
+        raise RuntimeError("query_start_loc must be contiguous int32")
     B = seq_lens.shape[0]
-    _check(block_table.shape[0] >= B and query_start_loc.shape[0] >= B + 1,
-           "block_table / query_start_loc shorter than seq_lens")
+    if block_table.shape[0] < B or query_start_loc.shape[0] < B + 1:
+        raise RuntimeError("block_table / query_start_loc shorter than seq_lens")
     if q_abs_offset is not None:
         _cuda(q_abs_offset, "q_abs_offset")
         _check(q_abs_offset.dtype == torch.int32 and q_abs_offset.is_contiguous()
                and q_abs_offset.shape[0] >= B, "q_abs_offset must be int32 [B]")
     if out is None:
-        out = torch.empty((T, Hq, D), dtype=out_dtype or query.dtype, device=query.device)
-    _cuda(out, "out")
-    _check(out.dtype in _DT and out.dim() == 3 and tuple(out.shape[1:]) == (Hq, D)
-           and out.shape[0] >= T and out.stride(2) == 1, "out must be [num_tokens, Hq, 128] fp32/fp16/bf16")
-    need = workspace_size(B, T, Hq, Hkv, max_query_len, max_seq_len)
+        out = torch.empty((T, Hq, D), dtype=out_dtype or query.dtype, device=dev)
+    odt = _DT.get(out.dtype)
+    if not out.is_cuda:
+        _cuda(out, "out")
+    oshape, ostrides = out.shape, out.stride()
+    if odt is None or len(oshape) != 3 or oshape[1] != Hq or oshape[2] != D or oshape[0] < T or ostrides[2] != 1:
+        raise RuntimeError("out must be [num_tokens, Hq, 128] fp32/fp16/bf16")
+    L = _load()
+    need = L.gfx906_fa_amd_paged_attention_workspace_size(B, T, Hq, Hkv, D, max_query_len, max_seq_len)
     if workspace is None:
-        workspace = new_workspace(need, query.device)
-    elif workspace.numel() * workspace.element_size() < need:
+        workspace = new_workspace(need, dev)
+    ws_bytes = workspace.nbytes
+    if ws_bytes < need:
         # the prefill tile-image room is optional: a workspace with the regions
         # every call needs runs as given (its prefill workgroups dequantize)
-        have = workspace.numel() * workspace.element_size()
-        if have < plan_info(B, T, Hq, Hkv, max_query_len, max_seq_len, D)["img_offset"]:
-            workspace = new_workspace(need, query.device)
-    _check(workspace.data_ptr() % 256 == 0, "workspace must be 256-byte aligned")
-    ws_bytes = workspace.numel() * workspace.element_size()
+        if ws_bytes < plan_info(B, T, Hq, Hkv, max_query_len, max_seq_len, D)["img_offset"]:
+            workspace = new_workspace(need, dev)
+            ws_bytes = workspace.nbytes
+    ws_ptr = workspace.data_ptr()
+    if ws_ptr % 256:
+        raise RuntimeError("workspace must be 256-byte aligned")
     if new_key is not None or new_value is not None or slot_mapping is not None:
         _check(new_key is not None and new_value is not None and slot_mapping is not None,
                "new_key, new_value and slot_mapping go together")
@@ -528,24 +572,23 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
         _check(new_key.stride(2) == 1 and new_value.stride(2) == 1, "new_key / new_value rows must be contiguous")
         _check(slot_mapping.dtype == torch.int64 and slot_mapping.shape[0] >= T, "slot_mapping must be int64 [T]")
         sm = slot_mapping.contiguous()
-        err = _load().gfx906_fa_amd_paged_attention_kv_write(
-            _ptr(query), _DT[query.dtype], query.stride(0), query.stride(1), _ptr(key_cache),
-            _ptr(value_cache), cbs, chs, _ptr(block_table), block_table.stride(0), _ptr(seq_lens),
-            _ptr(query_start_loc), _ptr(q_abs_offset), 1 if causal else 0, B, T, Hq, Hkv, D, bs,
-            int(max_query_len), int(max_seq_len), float(scale), _ptr(out), _DT[out.dtype],
-            out.stride(0), out.stride(1), _ptr(workspace), ws_bytes, _ptr(new_key), _ptr(new_value),
-            _DT[new_key.dtype], new_key.stride(0), new_key.stride(1), new_value.stride(0), new_value.stride(1),
-            _ptr(sm), _stream(query.device))
-        _ok(err, "gfx906_fa_amd_paged_attention_kv_write")
+        err = L.gfx906_fa_amd_paged_attention_kv_write(
+            query.data_ptr(), qdt, qts, qhs, key_cache.data_ptr(), value_cache.data_ptr(), cbs, chs,
+            block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), query_start_loc.data_ptr(),
+            _ptr(q_abs_offset), 1 if causal else 0, B, T, Hq, Hkv, D, bs, int(max_query_len), int(max_seq_len),
+            float(scale), out.data_ptr(), odt, ostrides[0], ostrides[1], ws_ptr, ws_bytes, new_key.data_ptr(),
+            new_value.data_ptr(), qdt, new_key.stride(0), new_key.stride(1), new_value.stride(0), new_value.stride(1),
+            sm.data_ptr(), _stream(dev))
+        if err:
+            _ok(err, "gfx906_fa_amd_paged_attention_kv_write")
         return out
-    err = _load().gfx906_fa_amd_paged_attention(
-        _ptr(query), _DT[query.dtype], query.stride(0), query.stride(1), _ptr(key_cache),
-        _ptr(value_cache), cbs, chs, _ptr(block_table), block_table.stride(0), _ptr(seq_lens),
-        _ptr(query_start_loc), _ptr(q_abs_offset), 1 if causal else 0, B, T, Hq, Hkv, D, bs,
-        int(max_query_len), int(max_seq_len), float(scale), _ptr(out), _DT[out.dtype],
-        out.stride(0), out.stride(1), _ptr(workspace), ws_bytes,
-        _stream(query.device))
-    _ok(err, "gfx906_fa_amd_paged_attention")
+    err = L.gfx906_fa_amd_paged_attention(
+        query.data_ptr(), qdt, qts, qhs, key_cache.data_ptr(), value_cache.data_ptr(), cbs, chs,
+        block_table.data_ptr(), block_table.stride(0), seq_lens.data_ptr(), query_start_loc.data_ptr(),
+        _ptr(q_abs_offset), 1 if causal else 0, B, T, Hq, Hkv, D, bs, int(max_query_len), int(max_seq_len),
+        float(scale), out.data_ptr(), odt, ostrides[0], ostrides[1], ws_ptr, ws_bytes, _stream(dev))
+    if err:
+        _ok(err, "gfx906_fa_amd_paged_attention")
     return out
 
 
@@ -584,8 +627,9 @@ def forward(q: torch.Tensor, k_q8: torch.Tensor, v_fp16: torch.Tensor, scale: fl
     shapes dequantize K and V once per call into tile images and run the tiled
     prefill kernel over them, long row tiles split over the keys."""
     for t, n in ((q, "q"), (k_q8, "k_q8"), (v_fp16, "v_fp16")):
-        _cuda(t, n)
-        _check(t.is_contiguous(), f"{n} must be contiguous")
+        if not t.is_cuda or not t.is_contiguous():
+            _cuda(t, n)
+            raise RuntimeError(f"{n} must be contiguous")
     _check(q.dtype == torch.float32, "q must be fp32")
     _check(k_q8.dtype == torch.uint8, "k_q8 must be uint8 (block_q8_0 bytes)")
     _check(v_fp16.dtype == torch.float16, "v_fp16 must be fp16")
@@ -599,8 +643,10 @@ def forward(q: torch.Tensor, k_q8: torch.Tensor, v_fp16: torch.Tensor, scale: fl
     _check(k_q8.dim() == 4 and tuple(k_q8.shape[:3]) == (B, Hkv, Skv),
            "k_q8 first 3 dims must match [B, Hkv, Skv]")
     _check(k_q8.shape[3] == D // QK8_0 * Q8_0_BYTES, "k_q8 last dim = (D/32)*34 bytes")
-    _check(D == 128, f"head_dim={D} unsupported (only 128)")
-    _check(Hq % Hkv == 0, f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
+    if D != 128:
+        raise RuntimeError(f"head_dim={D} unsupported (only 128)")
+    if Hq % Hkv:
+        raise RuntimeError(f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
     _check(mask is None or mask.dim() != 3 or mask.shape[2] >= Skv, "mask.size(2) must be >= seq_kv")
     mk, mbs, mrs, mcols = _mask_args(mask, B, Sq, q_abs_offset)
     dev = q.device
@@ -656,7 +702,8 @@ def forward_paged_direct(q: torch.Tensor, key_cache_q8: torch.Tensor, value_cach
     if B * Sq == 0:  # no query rows
         return out
     bs, Hkv, cbs, chs = _plane_info(key_cache_q8, value_cache)
-    _check(Hq % Hkv == 0, f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
+    if Hq % Hkv:
+        raise RuntimeError(f"heads_q={Hq} must be divisible by heads_kv={Hkv}")
     _check(bt.dim() == 2, "block_table must be int32 [num_seqs, max_blocks] with contiguous rows")
     if q_abs_offset is not None:
         _cuda(q_abs_offset, "q_abs_offset")

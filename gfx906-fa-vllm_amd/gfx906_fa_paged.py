@@ -140,7 +140,7 @@ def forward_paged(
         bt = bt.contiguous()
     o3 = None
     if out is not None:
-        o3 = out.view(out.shape[0], Hq, D)
+        o3 = out if out.dim() == 3 and out.shape[1] == Hq and out.shape[2] == D else out.view(out.shape[0], Hq, D)
     if _DBG:
         _fwdlog(f"forward_paged VARLEN: num_tokens={num_tokens} Hq={Hq} Hkv={key_cache.shape[1]} D={D} "
                 f"num_seqs={sl.shape[0]} Sq_max={max_seqlen_q} Sk_max={max_seqlen_k} "
