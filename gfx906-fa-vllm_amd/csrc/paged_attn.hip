@@ -109,8 +109,8 @@ struct AttnParams {
     void *out;
     int64_t o_ts, o_hs;
     float *ws_ml, *ws_o;  // partial (m, l) and O per slot row
-    int64_t *ws_hdr;      // decode plan published for the combine kernel: U, nwg
-    int *ws_pre;          // per-sequence exclusive prefix of decode sub-pages
+    int64_t *ws_hdr;      // decode plan published for the merge kernels (DecPlan)
+    int *ws_pre;          // per-sequence exclusive prefix of its pieces or units
     int num_seqs, nwg;    // nwg: decode workgroups (the grid)
     int dec_rows_lo;      // a decode launch takes sequences with dec_rows_lo < n_q*G
     int dec_rows_max;     //   <= dec_rows_max; the prefill kernel takes n_q*G > dec_rows_max
@@ -675,6 +675,12 @@ constexpr int DEC_CHUNK_ROWS = 64; // rows the two-row-group launch takes, in 32
 #ifndef GFA_DEC_MIN_UNITS
 #define GFA_DEC_MIN_UNITS 16
 #endif
+#ifndef GFA_DEC_ALIGN_SLACK
+#define GFA_DEC_ALIGN_SLACK 4
+#endif
+#ifndef GFA_DEC_ALIGN_UNITS
+#define GFA_DEC_ALIGN_UNITS 8  // sub-pages per piece of an aligned plan, at least
+#endif
 constexpr int DEC_MIN_UNITS = GFA_DEC_MIN_UNITS;  // sub-pages per decode workgroup, at least
 
 #ifndef GFA_DEC_DEPTH2
@@ -708,12 +714,20 @@ __device__ __forceinline__ SegInfo seg_info(const AttnParams &p, int s) {
     return si;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(v, o);
-        if (lane >= o) v += t;
-    }
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp_i32(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+
+// inclusive scan over the wave: shifts within each 16-lane DPP row, then the
+// rows' totals broadcast to the rows after them
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += dpp_i32<0x111>(v);       // row_shr:1
+    v += dpp_i32<0x112>(v);       // row_shr:2
+    v += dpp_i32<0x114>(v);       // row_shr:4
+    v += dpp_i32<0x118>(v);       // row_shr:8
+    v += dpp_i32<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp_i32<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
     return v;
 }
 
@@ -722,29 +736,103 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
            (uint32_t)__builtin_amdgcn_readfirstlane((int)(v & 0xFFFFFFFF));
 }
 
-// Total decode units U and the number of participating workgroups: at least
-// DEC_MIN_UNITS units per range, or one workgroup per segment where segments
-// are shorter than that (each piece a workgroup streams costs a Q load and a
-// cross-wave merge, so many short pieces in one range serialize), and at
-// most the resident workgroups.  Every range is non-empty: each counted
-// segment holds at least one unit.  Wave-level, uniform.
-__device__ __forceinline__ void dec_total(const AttnParams &p, int lane, int64_t &U, int &nwg) {
+// floor(a / b) for a >= 0, b >= 1.  Below 2^22 from the float quotient,
+// which is then within 1 of it, and one correction each way (the compiler's
+// integer division is a long instruction sequence).
+__device__ __forceinline__ int pl_div(int a, int b) {
+    if (a >= (1 << 22)) return a / b;
+    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    q += r < 0 ? -1 : (r >= b ? 1 : 0);
+    return q;
+}
+
+// How a decode launch's sub-pages are dealt to its workgroups, published in
+// the workspace for the merge kernels.
+//   aligned  (upw > 0, in 16ths of a sub-page; batches of up to 64 sequences)
+//            every segment is cut into ceil(16 nsub / upw) equal pieces, one
+//            workgroup each.
+//   stream-K (upw == 0) workgroup w takes units [Uv w / nwg, Uv (w+1) / nwg) of
+//            the segments laid end to end, each `pad` units of start-up
+//            followed by its nsub sub-pages: a piece's start (metadata, Q,
+//            page ids and first sub-pages: three dependent round trips, then
+//            the cross-wave merge) costs about what `pad` sub-pages do, so a
+//            workgroup whose range runs on into another segment streams that
+//            much less.
+// Aligned is taken where its pieces fit the resident workgroups at the even
+// share of the sub-pages per workgroup, or at stream-K's share (start-up
+// included) and GFA_DEC_ALIGN_SLACK: then no workgroup pays two starts.  With
+// plain equal ranges, one workgroup in eight did: 3 x (900, 100, 33) at 48/8,
+// 6.1 us a workgroup at the median and 13.4 for the slowest; 8 x 2000, 8.4
+// and 11.2.
+struct DecPlan {
+    int64_t U, Uv;     // sub-pages; with the start-up units
+    int nwg, upw, pad;
+};
+constexpr int DEC_HDR = 5;  // int64 words: U, nwg, upw, Uv, pad
+
+// Units per workgroup: at least DEC_MIN_UNITS, or one workgroup per segment
+// where segments are shorter than that; at most the resident workgroups.
+// Every range is non-empty.
+__device__ __forceinline__ int dec_nwg(const AttnParams &p, int64_t Uv, int nseg) {
+    const int64_t want = max(Uv / DEC_MIN_UNITS, (int64_t)nseg * p.Hkv);
+    return (int)max((int64_t)1, min((int64_t)p.nwg, want));
+}
+
+// The stream-K plan of a larger batch.  Wave-level, uniform.
+__device__ __forceinline__ DecPlan dec_total(const AttnParams &p, int lane, int pad) {
     int64_t tot = 0;
     int nseg = 0;
     for (int base = 0; base < p.num_seqs; base += 64) {
         const int si = base + lane;
         const int n = si < p.num_seqs ? seg_info(p, si).nsub : 0;
-        tot += __shfl(wave_incl_scan(n, lane), 63);
+        tot += __shfl(wave_incl_scan(n), 63);
         nseg += __builtin_popcountll(__ballot(n > 0));
     }
-    U = uniform64(tot * p.Hkv);
-    const int64_t want = max(U / DEC_MIN_UNITS, (int64_t)nseg * p.Hkv);
-    nwg = (int)max((int64_t)1, min((int64_t)p.nwg, want));
+    DecPlan d;
+    d.U = uniform64(tot * p.Hkv);
+    d.Uv = d.U + (int64_t)pad * nseg * p.Hkv;
+    d.pad = pad;
+    d.upw = 0;
+    d.nwg = dec_nwg(p, d.Uv, nseg);
+    return d;
 }
 
 __device__ __forceinline__ int64_t range_start(int64_t U, int k, int n) { return U * k / n; }
 // the workgroup whose range holds unit u
 __device__ __forceinline__ int range_of(int64_t U, int64_t u, int n) { return (int)(((u + 1) * n - 1) / U); }
+
+// The pieces of segment (s, h) as the merge kernels see them: workgroups wf ..
+// wl, each with its partial in slot 2k (the workgroup's first piece), or
+// 2k + 1 for wf when `odd` (its last piece).  One workgroup: written out.
+struct SegPieces {
+    int wf, wl;
+    bool odd;
+};
+__device__ __forceinline__ DecPlan load_plan(const AttnParams &p) {
+    DecPlan d;
+    d.U = p.ws_hdr[0];
+    d.nwg = (int)p.ws_hdr[1];
+    d.upw = (int)p.ws_hdr[2];
+    d.Uv = p.ws_hdr[3];
+    d.pad = (int)p.ws_hdr[4];
+    return d;
+}
+__device__ __forceinline__ SegPieces seg_pieces(const DecPlan &d, int pre, int Hkv, int h, int nsub) {
+    SegPieces sp;
+    if (d.upw > 0) {
+        const int c = pl_div(16 * nsub + d.upw - 1, d.upw);
+        sp.wf = pre * Hkv + h * c;
+        sp.wl = sp.wf + c - 1;
+        sp.odd = false;
+    } else {
+        const int64_t S0 = (int64_t)pre * Hkv + (int64_t)h * (nsub + d.pad);
+        sp.wf = range_of(d.Uv, S0 + d.pad, d.nwg);
+        sp.wl = range_of(d.Uv, S0 + d.pad + nsub - 1, d.nwg);
+        sp.odd = range_start(d.Uv, sp.wf, d.nwg) < S0;
+    }
+    return sp;
+}
 
 // CHUNK: sequences may have more rows than one tile (up to dec_rows_max):
 // each piece is streamed once per R-row chunk.  A separate instantiation, so
@@ -757,6 +845,17 @@ __device__ __forceinline__ int range_of(int64_t U, int64_t u, int n) { return (i
 // (the fused cache write of a decode step; 14 spilled VGPRs), and the
 // two-chunk mode pairs its waves two by two.
 constexpr int dec_nw(int nrg, bool chunk) { return nrg == 2 && !chunk ? 8 : DEC_NW; }
+
+// Start-up units of a segment (see DecPlan): the start takes 3 to 5 us, in
+// which a workgroup streams 2.3 sub-pages a microsecond with one row group (4
+// waves, three workgroups a CU), 5.4 as an 8-wave verify workgroup.
+#ifndef GFA_DEC_PAD
+#define GFA_DEC_PAD 16
+#endif
+#ifndef GFA_DEC_PAD8
+#define GFA_DEC_PAD8 32
+#endif
+constexpr int dec_pad(int nrg, bool chunk) { return nrg == 2 && !chunk ? GFA_DEC_PAD8 : GFA_DEC_PAD; }
 
 template <int NRG, int QDT, int ODT, bool CHUNK = false>
 __global__ __launch_bounds__(64 * dec_nw(NRG, CHUNK))
@@ -776,60 +875,100 @@ __attribute__((amdgpu_waves_per_eu(DecCfg<NRG>::wpe, DecCfg<NRG>::wpe))) void at
     // general path below takes three before the first K/V load.
     const bool small = B <= 64;
     SegInfo lsi = seg_info(p, small ? min(lane, B - 1) : 0);
+    constexpr int PAD = dec_pad(NRG, CHUNK);
     const int ln = small && lane < B ? lsi.nsub : 0;
-    const int lincl = wave_incl_scan(ln, lane);
-    int64_t U;
-    int nwg;
+    const int lv = ln > 0 ? ln + PAD : 0;  // with the start-up units
+    const int lincl = wave_incl_scan(lv);
+    DecPlan d;
+    int lc = 0, cincl = 0;  // aligned: pieces of sequence `lane` (per kv-head), and their prefix
     if (small) {
-        const int64_t tot = __shfl(lincl, 63);
         const int nseg = __builtin_popcountll(__ballot(ln > 0));
-        U = uniform64(tot * Hkv);
-        const int64_t want = max(U / DEC_MIN_UNITS, (int64_t)nseg * Hkv);
-        nwg = (int)max((int64_t)1, min((int64_t)p.nwg, want));
+        const int64_t tot = (int64_t)__builtin_amdgcn_readlane(lincl, 63) - (int64_t)PAD * nseg;
+        d.U = uniform64(tot * Hkv);
+        d.Uv = d.U + (int64_t)PAD * nseg * Hkv;
+        d.pad = PAD;
+        d.upw = 0;
+        d.nwg = dec_nwg(p, d.Uv, nseg);
+        const int maxc = p.nwg / Hkv;  // pieces of all sequences, at most
+        if (nseg > 0 && nseg <= maxc && tot < (1 << 24)) {
+            // the even share (in floats: one too few only costs a try), then
+            // what stream-K would give each workgroup, and a little
+            const float even = 16.0f * (float)tot / (float)maxc;
+            int upw = max((int)ceilf(even), 16 * GFA_DEC_ALIGN_UNITS);
+            for (int t = 0; t < 2 && d.upw == 0; ++t) {
+                lc = ln > 0 ? pl_div(16 * ln + upw - 1, upw) : 0;
+                cincl = wave_incl_scan(lc);
+                const int n = __builtin_amdgcn_readlane(cincl, 63);
+                if (n <= maxc) {
+                    d.upw = upw;
+                    d.nwg = n * Hkv;
+                }
+                upw = (int)(even + 16.0f * (float)(PAD * nseg) / (float)maxc) + 16 * GFA_DEC_ALIGN_SLACK;
+            }
+        }
     } else {
-        dec_total(p, lane, U, nwg);
+        d = dec_total(p, lane, PAD);
     }
+    const int64_t U = d.U;
     if (w == 0 && wv == 0) {
-        // publish the plan for attn_combine_kernel: U, nwg, per-sequence
-        // exclusive prefix of decode sub-pages
+        // publish the plan for the merge kernels: the header, and the
+        // per-sequence exclusive prefix of pieces (aligned) or of units
         if (small) {
-            if (lane < B) p.ws_pre[lane] = lincl - ln;
+            if (lane < B) p.ws_pre[lane] = d.upw ? cincl - lc : lincl - lv;
         } else {
             int64_t run = 0;
             for (int base = 0; base < B; base += 64) {
                 const int sj = base + lane;
-                const int n = sj < B ? seg_info(p, sj).nsub : 0;
-                const int incl = wave_incl_scan(n, lane);
+                const int nj = sj < B ? seg_info(p, sj).nsub : 0;
+                const int n = nj > 0 ? nj + PAD : 0;
+                const int incl = wave_incl_scan(n);
                 if (sj < B) p.ws_pre[sj] = (int)run + incl - n;
                 run += __shfl(incl, 63);
             }
         }
         if (lane == 0) {
-            p.ws_hdr[0] = U;
-            p.ws_hdr[1] = nwg;
+            p.ws_hdr[0] = d.U;
+            p.ws_hdr[1] = d.nwg;
+            p.ws_hdr[2] = d.upw;
+            p.ws_hdr[3] = d.Uv;
+            p.ws_hdr[4] = d.pad;
         }
     }
-    if (w >= nwg || U == 0) return;  // uniform over the workgroup
-    const int64_t u0 = range_start(U, w, nwg), u1 = range_start(U, w + 1, nwg);
+    if (w >= d.nwg || U == 0) return;  // uniform over the workgroup
+    int64_t u0 = 0, u1 = 0;
+    if (d.upw == 0) {
+        u0 = range_start(d.Uv, w, d.nwg);
+        u1 = range_start(d.Uv, w + 1, d.nwg);
+    }
     // locate the sequence holding u0 (Ps = sub-pages of the sequences before s)
     int s = 0;
     int64_t Ps = 0;
     SegInfo si;
     if (small) {
-        const uint64_t bal = __ballot((int64_t)lincl * Hkv > u0);  // non-empty: u0 < U
+        const uint64_t bal = d.upw ? __ballot(cincl * Hkv > w) : __ballot((int64_t)lincl * Hkv > u0);  // non-empty
         s = __builtin_ctzll(bal);
-        Ps = __builtin_amdgcn_readlane(lincl - ln, s);
+        Ps = __builtin_amdgcn_readlane(lincl - lv, s);
         si.q0 = __builtin_amdgcn_readlane(lsi.q0, s);
         si.nq = __builtin_amdgcn_readlane(lsi.nq, s);
         si.sl = __builtin_amdgcn_readlane(lsi.sl, s);
         si.qa = __builtin_amdgcn_readlane(lsi.qa, s);
         si.kv_lim = __builtin_amdgcn_readlane(lsi.kv_lim, s);
         si.nsub = __builtin_amdgcn_readlane(lsi.nsub, s);
+        if (d.upw) {  // piece j of c of kv-head h: sub-pages [j nsub / c, (j + 1) nsub / c)
+            const int c = __builtin_amdgcn_readlane(lc, s);
+            const int r = w - __builtin_amdgcn_readlane(cincl - lc, s) * Hkv;
+            const int h = pl_div(r, c), j = r - h * c;
+            const int q = pl_div(si.nsub, c), rem = si.nsub - q * c;
+            const int a = j * q + pl_div(j * rem, c), b = (j + 1) * q + pl_div((j + 1) * rem, c);
+            u0 = Ps * Hkv + (int64_t)h * (si.nsub + PAD) + PAD + a;
+            u1 = u0 + (b - a);
+        }
     } else {
         for (int base = 0; base < B; base += 64) {
             const int sidx = base + lane;
-            const int n = sidx < B ? seg_info(p, sidx).nsub : 0;
-            const int incl = wave_incl_scan(n, lane);
+            const int nj = sidx < B ? seg_info(p, sidx).nsub : 0;
+            const int n = nj > 0 ? nj + PAD : 0;
+            const int incl = wave_incl_scan(n);
             const int ctot = __shfl(incl, 63);
             if ((Ps + ctot) * Hkv > u0) {
                 const uint64_t bal = __ballot((Ps + incl) * Hkv > u0);
@@ -859,9 +998,10 @@ __attribute__((amdgpu_waves_per_eu(DecCfg<NRG>::wpe, DecCfg<NRG>::wpe))) void at
         SegInfo sv = si;
         while (uu < u1) {
             const int64_t off = uu - Pw * Hkv;
-            const int hh = (int)(off / sv.nsub);
-            const int a = (int)(off - (int64_t)hh * sv.nsub);
-            const int b = (int)min((int64_t)sv.nsub, a + (u1 - uu));
+            const int nv = sv.nsub + PAD;
+            const int hh = off < (1 << 22) ? pl_div((int)off, nv) : (int)(off / nv);
+            const int av = (int)(off - (int64_t)hh * nv), bv = (int)min((int64_t)nv, av + (u1 - uu));
+            const int a = max(av - PAD, 0), b = bv - PAD;  // (b <= a: start-up units only)
             const int lo = sv.sl - sv.nq;
             // two row chunks at once (see rows_pass below): sub-page js is
             // streamed by the two waves with (js - a) % 2 == wv % 2, and both
@@ -873,9 +1013,9 @@ __attribute__((amdgpu_waves_per_eu(DecCfg<NRG>::wpe, DecCfg<NRG>::wpe))) void at
                 for (int pos = max(16 * js, lo); pos < t_hi; ++pos)
                     write_new_token<QDT>(p, hh, sv.q0 + (pos - lo), lane);
             }
-            uu += b - a;
-            if (uu < u1 && b == sv.nsub && hh == Hkv - 1) {
-                Pw += sv.nsub;
+            uu += bv - av;
+            if (uu < u1 && bv == nv && hh == Hkv - 1) {
+                Pw += nv;
                 do {
                     ++sw;
                     sv = seg_info(p, sw);
@@ -899,9 +1039,10 @@ __attribute__((amdgpu_waves_per_eu(DecCfg<NRG>::wpe, DecCfg<NRG>::wpe))) void at
     bool first = true;
     while (u < u1) {
         const int64_t off = u - Ps * Hkv;
-        const int h = (int)(off / si.nsub);
-        const int a = (int)(off - (int64_t)h * si.nsub);
-        const int b = (int)min((int64_t)si.nsub, a + (u1 - u));
+        const int nv = si.nsub + PAD;
+        const int h = off < (1 << 22) ? pl_div((int)off, nv) : (int)(off / nv);
+        const int av = (int)(off - (int64_t)h * nv), bv = (int)min((int64_t)nv, av + (u1 - u));
+        const int a = max(av - PAD, 0), b = bv - PAD;  // (b <= a: start-up units only)
         const int nrows = si.nq * p.G;
 
         // CHUNK: rows beyond one tile (up to 64: a verify step of 6 tokens at
@@ -989,15 +1130,17 @@ __attribute__((amdgpu_waves_per_eu(DecCfg<NRG>::wpe, DecCfg<NRG>::wpe))) void at
         }
         };
         static_assert((NW == 4 || !CHUNK) && DEC_CHUNK_ROWS <= 2 * 32, "two row chunks of two waves each");
-        if (CHUNK && nrows > R) {  // uniform: rows R..nrows-1 (nrows <= 2R) in the second chunk
-            rows_pass(R * (wv >> 1), wv & 1, 2, NW / 2);
-        } else {
-            rows_pass(0, wv, NW, NW);
+        if (b > a) {  // uniform
+            if (CHUNK && nrows > R) {  // uniform: rows R..nrows-1 (nrows <= 2R) in the second chunk
+                rows_pass(R * (wv >> 1), wv & 1, 2, NW / 2);
+            } else {
+                rows_pass(0, wv, NW, NW);
+            }
+            first = false;
         }
-        u += b - a;
-        first = false;
-        if (u < u1 && b == si.nsub && h == Hkv - 1) {  // next sequence with decode work
-            Ps += si.nsub;
+        u += bv - av;
+        if (u < u1 && bv == nv && h == Hkv - 1) {  // next sequence with decode work
+            Ps += nv;
             do {
                 ++s;
                 si = seg_info(p, s);
@@ -1025,16 +1168,14 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     // the plan words are read together with the sequence's metadata (one
     // memory round trip instead of two: they are needed only when the
     // segment turns out to be split)
-    const int64_t U = p.ws_hdr[0];
-    const int nwg = (int)p.ws_hdr[1];
+    const DecPlan d = load_plan(p);
     const int pre = p.ws_pre[s];
     const SegInfo si = seg_info(p, s);
     if (si.nsub == 0 || r >= si.nq * p.G) return;
-    if (U == 0) return;
-    const int64_t S0 = (int64_t)pre * p.Hkv + (int64_t)h * si.nsub;
-    const int wf = range_of(U, S0, nwg), wl = range_of(U, S0 + si.nsub - 1, nwg);
-    if (wf == wl && range_start(U, wf, nwg) <= S0 && range_start(U, wf + 1, nwg) >= S0 + si.nsub)
-        return;  // whole segment in one workgroup: already written
+    if (d.U == 0) return;
+    const SegPieces sp = seg_pieces(d, pre, p.Hkv, h, si.nsub);
+    const int wf = sp.wf, wl = sp.wl;
+    if (wf == wl) return;  // whole segment in one workgroup: already written
     const int t = threadIdx.x, dc = t & 31, sub = t >> 5;
     const int d0 = 4 * dc;
     float m = -INFINITY, l = 0.f;
@@ -1052,7 +1193,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
         for (int i = 0; i < CU; ++i) {
             const int k = k0 + 8 * i;
             if (k <= wl) {
-                const int sk = (k == wf && range_start(U, k, nwg) < S0) ? 2 * k + 1 : 2 * k;
+                const int sk = (k == wf && sp.odd) ? 2 * k + 1 : 2 * k;
                 const int64_t row = (int64_t)sk * p.dec_rows_max + r;
                 mlk[i] = *reinterpret_cast<const float2_t *>(p.ws_ml + 2 * row);
                 ok[i] = *reinterpret_cast<const float4_t *>(p.ws_o + row * 128 + d0);
@@ -1106,15 +1247,13 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
 template <int ODT>
 __global__ __launch_bounds__(256) void attn_combine_few_kernel(AttnParams p) {
     const int s = blockIdx.x, h = blockIdx.y;
-    const int64_t U = p.ws_hdr[0];
-    const int nwg = (int)p.ws_hdr[1];
+    const DecPlan d = load_plan(p);
     const int pre = p.ws_pre[s];
     const SegInfo si = seg_info(p, s);
-    if (si.nsub == 0 || U == 0) return;
-    const int64_t S0 = (int64_t)pre * p.Hkv + (int64_t)h * si.nsub;
-    const int wf = range_of(U, S0, nwg), wl = range_of(U, S0 + si.nsub - 1, nwg);
-    if (wf == wl && range_start(U, wf, nwg) <= S0 && range_start(U, wf + 1, nwg) >= S0 + si.nsub)
-        return;  // whole segment in one workgroup: already written
+    if (si.nsub == 0 || d.U == 0) return;
+    const SegPieces sp = seg_pieces(d, pre, p.Hkv, h, si.nsub);
+    const int wf = sp.wf, wl = sp.wl;
+    if (wf == wl) return;  // whole segment in one workgroup: already written
     const int rows = si.nq * p.G;
     const int dc = threadIdx.x & 31, d0 = 4 * dc;
     constexpr int CU = 8;
@@ -1128,7 +1267,7 @@ __global__ __launch_bounds__(256) void attn_combine_few_kernel(AttnParams p) {
             for (int i = 0; i < CU; ++i) {
                 const int k = k0 + i;
                 if (k <= wl) {
-                    const int sk = (k == wf && range_start(U, k, nwg) < S0) ? 2 * k + 1 : 2 * k;
+                    const int sk = (k == wf && sp.odd) ? 2 * k + 1 : 2 * k;
                     const int64_t row = (int64_t)sk * p.dec_rows_max + r;
                     mlk[i] = *reinterpret_cast<const float2_t *>(p.ws_ml + 2 * row);
                     ok[i] = *reinterpret_cast<const float4_t *>(p.ws_o + row * 128 + d0);
@@ -2043,11 +2182,6 @@ constexpr int PF_SPLIT_MIN = GFA_PF_SPLIT_MIN;  // a split row tile's pieces: at
 #define GFA_PFC_WGS_PER_CU 4  // split-merge workgroups per CU (more loads in flight)
 #endif
 
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ int dpp_i32(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
-}
-
 // sum over the wave, every lane receives it: butterflies within each 16-lane
 // DPP row, then across the four rows with the permlane swaps
 __device__ __forceinline__ int pl_wave_sum32(int v) {
@@ -2073,24 +2207,12 @@ __device__ __forceinline__ int pl_wave_max32(int v) {
     return max((int)b[0], (int)b[1]);
 }
 
-// inclusive scan over the wave: shifts within each 16-lane DPP row, then the
-// rows' totals broadcast to the rows after them
-__device__ __forceinline__ int pl_wave_scan32(int v) {
-    v += dpp_i32<0x111>(v);       // row_shr:1
-    v += dpp_i32<0x112>(v);       // row_shr:2
-    v += dpp_i32<0x114>(v);       // row_shr:4
-    v += dpp_i32<0x118>(v);       // row_shr:8
-    v += dpp_i32<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
-    v += dpp_i32<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
 // exclusive scan of v over the workgroup; *total receives the sum (a scan
 // inside each wave, then the waves' totals through tmp)
 __device__ __forceinline__ int pl_block_scan(int v, int *tmp, int *total) {
     constexpr int NT = PL_THREADS;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int x = pl_wave_scan32(v);
+    const int x = wave_incl_scan(v);
     __syncthreads();  // tmp[] of a previous call has been read
     if (lane == 63) tmp[wv] = x;
     __syncthreads();
@@ -2103,17 +2225,6 @@ __device__ __forceinline__ int pl_block_scan(int v, int *tmp, int *total) {
     }
     *total = tot;
     return before + x - v;
-}
-
-// floor(a / b) for a >= 0, b >= 1.  Below 2^22 from the float quotient,
-// which is then within 1 of it, and one correction each way (the compiler's
-// integer division is a long instruction sequence).
-__device__ __forceinline__ int pl_div(int a, int b) {
-    if (a >= (1 << 22)) return a / b;
-    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
-    const int r = a - q * b;
-    q += r < 0 ? -1 : (r >= b ? 1 : 0);
-    return q;
 }
 
 // A sequence's scalars as the plan reads them.
@@ -2443,14 +2554,14 @@ __global__ __launch_bounds__(64) void prefill_plan_wave_kernel(AttnParams p) {
     const PlSeq qs = pl_seq(p, sq0);
     const int q0s = seq_q0(p, sq0);
     const int v = lane < B ? pl_tiles(p, qs) : 0;
-    const int pre = pl_wave_scan32(v);  // inclusive
+    const int pre = wave_incl_scan(v);  // inclusive
     const int n = min(min(rl(pre, 63), p.pf_items_max), PW_MAX);
     int icarry = 0;
     if (p.pf_tbase != nullptr) {
         // first image tile of each sequence (see the general kernel)
         const int vt = v > 0 ? pl_ntk(p, qs, v - 1) : 0;
         const bool big = pl_wave_max32(vt) > (1 << 20);
-        const int it = pl_wave_scan32(min(vt, 1 << 20));
+        const int it = wave_incl_scan(min(vt, 1 << 20));
         if (lane < B) p.pf_tbase[lane] = it - min(vt, 1 << 20);
         if (lane == 0) p.pf_tbase[B] = rl(it, 63);
         icarry = big ? INT32_MAX : rl(it, 63);
@@ -2522,7 +2633,7 @@ __global__ __launch_bounds__(64) void prefill_plan_wave_kernel(AttnParams p) {
     }
     int k = act ? pl_pieces(w, tsplit) : 0;
     int total = pl_wave_sum32(k);
-    int ssum = pl_wave_scan32(k > 1 ? k : 0);
+    int ssum = wave_incl_scan(k > 1 ? k : 0);
     uint64_t smask = __ballot(k > 1);
     if (total > min(p.pf_grid_items, PW_PIECES) || rl(ssum, 63) > p.pf_slots_max ||
         __builtin_popcountll(smask) > p.pf_split_max) {  // past the workspace: nothing is cut
@@ -2541,7 +2652,7 @@ __global__ __launch_bounds__(64) void prefill_plan_wave_kernel(AttnParams p) {
     }
     // heaviest first, by the row tile's piece size (a row tile's pieces follow
     // each other); in any order where all run at once
-    const int at = total > m ? place(k > 0 ? pl_div(w + k - 1, k) : -1, k) : pl_wave_scan32(k) - k;
+    const int at = total > m ? place(k > 0 ? pl_div(w + k - 1, k) : -1, k) : wave_incl_scan(k) - k;
     if (pl_wave_max32(k) <= 16) {
         for (int c = 0; c < k; ++c) s_map[at + c] = (uint8_t)lane;
     } else {
