@@ -40,7 +40,8 @@ def test_noalloc_drops_the_work_list_before_refusing():
     on the 2-D grid, with the outputs of the workspace entry."""
     need_gpu()
     B, Hq, L = 8192, 16, 808
-    T = B * L - 1                                   # not uniform: the decode classes are laid out too
+    last = 3                                        # 48 rows: the decode classes are laid out too
+    T = (B - 1) * L + last
     info = gfx906_fa.plan_info(B, T, Hq, 1, L, L)
     base, items = info["pf_header_offset"] + 256, info["pf_grid_items"]
     # (the split partials are dropped first; 1 MiB of slack covers the small regions)
@@ -54,7 +55,7 @@ def test_noalloc_drops_the_work_list_before_refusing():
     gfx906_fa.reshape_and_cache_q8_kv(kv[0], kv[1], torch.arange(L, device=DEV), cache[:, 0], cache[:, 1])
     bt = torch.arange(nb, dtype=torch.int32, device=DEV).repeat(B, 1)  # every sequence reads the same pages
     lens = np.full(B, L, np.int32)
-    lens[-1] = L - 1
+    lens[-1] = last
     sl = torch.from_numpy(lens).to(DEV)
     qsl = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).to(DEV)
     q = torch.randn((T, Hq, 128), generator=g, device=DEV, dtype=torch.float16)
