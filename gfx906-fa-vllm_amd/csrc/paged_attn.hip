@@ -1605,6 +1605,30 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
                 if (h + 4 < 2 * ntk) __builtin_amdgcn_s_waitcnt(0x0F7F);  // vmcnt(15)
                 else __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
             };
+            // Images of contiguous inputs hold V rows as the caller has them, also
+            // of keys past kv_end, whose P = 0 does not cancel an Inf or a NaN:
+            // each wave clears them in its own share of the last tile's V^T
+            // stage (32 rows of 8 chunks, four 16-byte chunks a lane), once the
+            // share has landed.  (Paged images hold finite values, see
+            // pf_dequant_v.)  Chunk c: keys t0 .. t0 + 3 and t0 + 8 .. t0 + 11
+            // of the tile, t0 = 16 (c / 2) + 4 (c % 2).
+            static_assert(PF_VSHARE == 32 * PF_VPITCH && PF_TK == 64, "a V^T share: 32 rows of 64 keys");
+            const int nv_last = kv_end - PF_TK * (ktb + ntk - 1);  // keys of the last tile that a row may see
+            const bool clear = p.pf_img_seq > 0 && ntk > 0 && nv_last < PF_TK;
+            auto clear_unseen = [&]() __attribute__((always_inline)) {
+                uint8_t *const vst = ldsv + ((ntk - 1) % PF_NSTAGE) * PF_VBYTES + wsp * PF_VSHARE;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = lane & 7, t0 = 16 * (c >> 1) + 4 * (c & 1);
+                    uint64_t *const x = reinterpret_cast<uint64_t *>(vst + ((lane >> 3) + 8 * i) * PF_VPITCH + 16 * c);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int n = nv_last - (t0 + 8 * e);  // seen keys of the four
+                        if (n <= 0) x[e] = 0;
+                        else if (n < 4) x[e] &= (1ull << (16 * n)) - 1;
+                    }
+                }
+            };
             copy(0);
             first_loads_issued();
             copy(1);
@@ -1615,6 +1639,10 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             for (int hs = 0; hs <= 2 * ntk; ++hs) {  // half-steps 0 .. 2 ntk
                 copy(hs + 4);
                 landed(hs);
+                if (clear && hs == 2 * (ntk - 1)) {  // uniform: the last V^T stage has landed, and is read from hs + 1 on
+                    asm volatile("" ::: "memory");
+                    clear_unseen();
+                }
                 __syncthreads();
             }
             return;
