@@ -3276,6 +3276,7 @@ struct Plan {
     DecClass dc[3];
     int ndc;            // decode classes launched (0..3)
     int dec_rows_max;   // largest decode row bound (0: every sequence is prefill)
+    bool one_class;     // a mixed batch's one class for all decode row counts
     bool need_prefill;
     int pf_rows;        // rows per prefill row tile: PF_ROWS (KS = 1) or PF_ROWS / 2 (KS = 2)
     int pf_items_max;   // bound on prefill row tiles (0: no work list)
@@ -3417,9 +3418,11 @@ Plan make_plan(int num_seqs, int num_tokens, int num_heads, int num_kv_heads, in
     const int G = num_heads / num_kv_heads;
     const int max_rows = max_query_len * G;
     const bool uniform = (int64_t)num_tokens == (int64_t)num_seqs * max_query_len;
-    // query tokens of the shortest sequence, at least: no other has more than
-    // max_query_len (a sequence that is shorter after all runs as a prefill)
+    // query tokens of the shortest sequence, at least, where every query row
+    // belongs to a sequence: no other has more than max_query_len
     const int64_t n_min = (int64_t)num_tokens - (int64_t)(num_seqs - 1) * max_query_len;
+    // the query tensor has rows past the last sequence, for certain
+    const bool past_end = (int64_t)num_tokens > (int64_t)num_seqs * max_query_len;
     pl.ndc = 0;
     // tiles of 16, 32 or 48 rows per wave (one, two or three row groups);
     // up to DEC_CHUNK_ROWS rows the two-row-group class takes in 32-row
@@ -3439,12 +3442,22 @@ Plan make_plan(int num_seqs, int num_tokens, int num_heads, int num_kv_heads, in
     } else if (uniform) {
         if (rows48) plan_add_class(pl, 3, 0, 48);
         else if (max_rows <= DEC_CHUNK_ROWS) plan_add_class(pl, 2, 0, hi2);
-    } else if (n_min * G <= DEC_CHUNK_ROWS) {
+    } else if (n_min * G > DEC_CHUNK_ROWS && !past_end) {
+        // A few prompts of like lengths: even the shortest has more rows than
+        // the decode classes take, unless the query tensor has rows past the
+        // last sequence, which the host cannot rule out.  One class for every
+        // decode row count then stands in for the two below (two launches
+        // that find nothing instead of four: 1252 + 242 + 1070 tokens at 48/8
+        // 77.4 -> 64.8 us a call; without any, 60.2).  Without it, a decode
+        // beside such rows runs as a prefill: 512 + 1 tokens in 528 rows, the
+        // decode on 131072 keys, 64/8: 141 us, 82.2 with this class, 89.8 with
+        // the two.  From 4 to 30 decodes or verifies in such batches: 1.06 to
+        // 1.4 times as fast as with the two.
+        if (G <= DEC_CHUNK_ROWS) plan_add_class(pl, 2, 0, DEC_CHUNK_ROWS);
+        pl.one_class = true;
+    } else {
         // mixed row counts: each sequence takes the smallest tile that
-        // holds its rows (one launch pair per class).  Not where even the
-        // shortest sequence has more rows than the decode classes take (a few
-        // prompts of like lengths): four launches that would find nothing
-        // (1252 + 242 + 1070 tokens at 48/8: 77.5 -> 67.2 us a step).
+        // holds its rows (one launch pair per class)
         if (G <= 16) plan_add_class(pl, 1, 0, 16);
         if (rows48) {
             if (G <= 32) plan_add_class(pl, 2, pl.ndc ? 16 : 0, 32);
@@ -3573,7 +3586,9 @@ hipError_t launch_all(const AttnParams &p0, const Plan &pl, char *ws, int num_se
                 pd.nwg = c.nwg * DEC_NW / nw;
                 attn_decode_kernel<2, QDT, ODT><<<pd.nwg, 64 * nw, 0, stream>>>(pd);
             }
-            if (c.rows_lo > 0 && (int64_t)num_seqs * num_kv_heads >= GFA_COMB_SEGS)
+            // (a mixed batch's class mostly finds nothing to merge: 250 prompts
+            // of 30 tokens at 48/8 128 us with a launch per row, 89.5 per segment)
+            if ((c.rows_lo > 0 || pl.one_class) && (int64_t)num_seqs * num_kv_heads >= GFA_COMB_SEGS)
                 attn_combine_few_kernel<ODT><<<dim3(num_seqs, num_kv_heads), 256, 0, stream>>>(pd);
             else
                 attn_combine_kernel<2, ODT><<<dim3(num_seqs, num_kv_heads, crow), 256, 0, stream>>>(pd);
