@@ -672,6 +672,12 @@ __device__ __forceinline__ void write_new_token(const AttnParams &p, int h, int6
 
 constexpr int DEC_NW = 4;          // waves per decode workgroup
 constexpr int DEC_CHUNK_ROWS = 64; // rows the two-row-group launch takes, in 32-row chunks
+// Over 30 decode and verify batches of 1 to 63 sequences drawn over the path's
+// ranges, the plan's constants measured (geometric means against the values
+// here): ALIGN_SLACK 0 and 16 1.000 and 1.003, so the slack only has to be
+// there; ALIGN_UNITS 4 0.953 (a single sequence of 18K keys at 8/1 16.3 -> 22.1
+// us: more pieces to merge than they save), 16 1.005 (0.83 to 1.26: short
+// verifies lose what two or three long contexts gain).
 #ifndef GFA_DEC_MIN_UNITS
 #define GFA_DEC_MIN_UNITS 16
 #endif
@@ -681,7 +687,7 @@ constexpr int DEC_CHUNK_ROWS = 64; // rows the two-row-group launch takes, in 32
 #ifndef GFA_DEC_ALIGN_UNITS
 #define GFA_DEC_ALIGN_UNITS 8  // sub-pages per piece of an aligned plan, at least
 #endif
-constexpr int DEC_MIN_UNITS = GFA_DEC_MIN_UNITS;  // sub-pages per decode workgroup, at least
+constexpr int DEC_MIN_UNITS = GFA_DEC_MIN_UNITS;  // stream-K units per workgroup, at least (start-up units included)
 
 #ifndef GFA_DEC_DEPTH2
 #define GFA_DEC_DEPTH2 2
@@ -771,9 +777,15 @@ struct DecPlan {
 };
 constexpr int DEC_HDR = 5;  // int64 words: U, nwg, upw, Uv, pad
 
-// Units per workgroup: at least DEC_MIN_UNITS, or one workgroup per segment
-// where segments are shorter than that; at most the resident workgroups.
-// Every range is non-empty.
+// Workgroups of a stream-K plan of Uv units (start-up units included): at
+// least DEC_MIN_UNITS units each, or one workgroup per segment where that is
+// more; at most the resident workgroups.  Every range holds a unit, but with
+// segments shorter than their start-up a range may hold start-up units only,
+// and its workgroup streams nothing.  Counting sub-pages alone leaves fewer
+// workgroups and measured worse, as several short segments then queue in one
+// (this rule and that one: 65 x 13-21 keys, 5 verify tokens, 6/1, 14.8 and
+// 19.0 us; 128 x 38-305, 20.1 and 22.9; over 83 batches of 65 to 512
+// sequences that one is 2 % slower in the geometric mean).
 __device__ __forceinline__ int dec_nwg(const AttnParams &p, int64_t Uv, int nseg) {
     const int64_t want = max(Uv / DEC_MIN_UNITS, (int64_t)nseg * p.Hkv);
     return (int)max((int64_t)1, min((int64_t)p.nwg, want));
@@ -2551,6 +2563,11 @@ __global__ __launch_bounds__(PL_THREADS) void prefill_plan_kernel(AttnParams p) 
 // 1252 + 242 + 1070 fresh tokens 80.2 -> 77.2 (not split; the plan itself 8.2
 // -> 7.6 us there, 7.0 -> 4.0 us with 4 row tiles).  Pieces of 4 tiles and up
 // were within 1 us of these, and 2 us worse where 5 key tiles were cut.
+// The constants, over 24 batches of 1 to 6 prompts (fresh and on prefixes) and
+// 12 contiguous calls drawn over the path's ranges (geometric means against
+// the values here): START 2 and 8 1.009 and 1.002, PART 4 and 16 1.008 and
+// 0.999, SPLIT_MIN 4 and 10 1.017 and 1.009 (4: contiguous calls of 400 to
+// 1000 keys 1.04 to 1.14, paged ones within noise; 10: from 0.91 to 1.06).
 #ifndef GFA_PW_START
 #define GFA_PW_START 4
 #endif
