@@ -139,7 +139,7 @@ struct AttnParams {
     // the prefill workgroups then copy them into LDS instead of dequantizing
     // every tile themselves.
     uint8_t *pf_tiles;
-    int pf_img_seq;     // > 0: images of every key tile are there, this many per sequence (flat attention)
+    int pf_img_seq;     // flat attention: images of every key tile are there, this many per sequence
     int *pf_tbase;      // per sequence (num_seqs + 1): first image tile
     int64_t pf_tiles_cap;
     // Fused cache write of the step's new tokens (decode kernels only; nullptr:
@@ -1522,10 +1522,15 @@ __device__ __forceinline__ void pf_dequant_v(const PfRaw &r, uint8_t *vst, int s
     }
 }
 
-template <int QDT, int ODT, bool VF16, bool MASK, int KS = 1>
+// FLAT: the tile images of contiguous inputs (pf_img_seq per sequence, all of
+// them there), whose V rows are the caller's own.  An instance of its own: the
+// clearing of unseen V in the paged instance's copy loop cost the 32K prompt
+// 1 % (11.07 -> 11.2 ms), though it never ran there.
+template <int QDT, int ODT, bool VF16, bool MASK, int KS = 1, bool FLAT = false>
 __global__ __launch_bounds__(64 * PF_WAVES)
 __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p) {
     static_assert(KS == 1 || KS == 2, "256-row tiles, or 128-row key-interleaved tiles");
+    static_assert(!FLAT || KS == 1, "images are for 256-row tiles");
     constexpr int ROWS = PF_ROWS / KS;               // query rows per tile
     constexpr int NSTAGE = KS == 1 ? PF_NSTAGE : 2;  // LDS stages of K^ and of V^T (tile t: t % NSTAGE)
     // (KS = 2 has room for the consumers' Q rows of its own; KS = 1 puts them
@@ -1582,7 +1587,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
         // fetch until its dequant, one iteration before the consumers read it.
         const int wsp = w - PF_CWAVES;
         // (no images for KS = 2 tiles: the host never passes them there)
-        if (KS == 1 && p.pf_tiles != nullptr && (p.pf_img_seq > 0 || p.pf_count[2] != 0)) {  // uniform
+        if (FLAT || (KS == 1 && p.pf_tiles != nullptr && p.pf_count[2] != 0)) {  // uniform
             // The tiles are dequantized images in the workspace.  Copy batch
             // b (K^ of tile b/2 for even b, V^T for odd b) goes from the image
             // straight into its LDS stage in half-step b - 4 and has landed by
@@ -1594,7 +1599,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             // batches may still be in flight), or vmcnt(0) near the end, where
             // fewer batches follow.
             const int64_t istride = (int64_t)Hkv * PF_IMG_BYTES;
-            const int64_t tb = p.pf_img_seq > 0 ? (int64_t)s * p.pf_img_seq : (int64_t)p.pf_tbase[s];
+            const int64_t tb = FLAT ? (int64_t)s * p.pf_img_seq : (int64_t)p.pf_tbase[s];
             const uint8_t *img0 = p.pf_tiles + ((tb + ktb) * Hkv + h) * PF_IMG_BYTES;
             auto copy = [&](int b) __attribute__((always_inline)) {
                 const int t = b >> 1;
@@ -1626,7 +1631,7 @@ __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_prefill_kernel(AttnParams p
             // of the tile, t0 = 16 (c / 2) + 4 (c % 2).
             static_assert(PF_VSHARE == 32 * PF_VPITCH && PF_TK == 64, "a V^T share: 32 rows of 64 keys");
             const int nv_last = kv_end - PF_TK * (ktb + ntk - 1);  // keys of the last tile that a row may see
-            const bool clear = p.pf_img_seq > 0 && ntk > 0 && nv_last < PF_TK;
+            const bool clear = FLAT && ntk > 0 && nv_last < PF_TK;
             auto clear_unseen = [&]() __attribute__((always_inline)) {
                 uint8_t *const vst = ldsv + ((ntk - 1) % PF_NSTAGE) * PF_VBYTES + wsp * PF_VSHARE;
 #pragma unroll
@@ -4207,8 +4212,10 @@ extern "C" hipError_t gfx906_fa_amd_flat_attention(
     if (p.pf_items) launch_plan(p, pl, batch, stream);
     const int tiles = (int)(((int64_t)seq_q * G + PF_ROWS - 1) / PF_ROWS);
     const dim3 grid = p.pf_items ? dim3(pl.pf_grid_items * num_kv_heads) : dim3(tiles * num_kv_heads, batch);
-    if (mask) attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
-    else attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, false><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+    if (mask)
+        attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, true, 1, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
+    else
+        attn_prefill_kernel<GFA_DTYPE_F32, GFA_DTYPE_F32, false, false, 1, true><<<grid, 64 * PF_WAVES, 0, stream>>>(p);
     if (p.pf_items && pl.pf_slots_max)
         attn_prefill_combine_kernel<GFA_DTYPE_F32><<<device_cus() * GFA_PFC_WGS_PER_CU, 256, 0, stream>>>(p);
     return hipGetLastError();
