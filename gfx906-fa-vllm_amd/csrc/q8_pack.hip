@@ -1,7 +1,7 @@
-// q8_pack.hip - contiguous -> planar repacking for the flat attention entry
-// (the op module's forward(), the reference's contiguous path
-// extension/gfx906_fa.cpp:120-265 over K_q8 [B, Hkv, Skv, 136] and fp16
-// V [B, Hkv, Skv, D]).
+// q8_pack.hip - contiguous -> planar repacking for the tiled attention entry
+// (the inputs of the reference's contiguous path, extension/gfx906_fa.cpp:120-265:
+// K_q8 [B, Hkv, Skv, 136] and fp16 V [B, Hkv, Skv, D]).  For callers of the C
+// ABI; the op module's forward() writes tile images instead.
 //
 //   pack_k_kernel    AoS Q8_0 K rows -> planar Q8 K sub-pages (a byte
 //                    permutation: the same Q8_0 blocks, placed for the MFMA

@@ -594,7 +594,7 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
 
 def _mask_args(mask: Optional[torch.Tensor], B: int, Sq: int, q_abs_offset):
     """fp16 additive mask [B, Sq, Skv_pad] (``extension/gfx906_fa.cpp:214-227``)
-    -> (tensor, batch stride, row stride, columns) for the tiled entry."""
+    -> (tensor, batch stride, row stride, columns) for the C entries."""
     if mask is None:
         return None, 0, 0, 0
     _check(q_abs_offset is None,

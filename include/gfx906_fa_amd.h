@@ -175,7 +175,9 @@ hipError_t gfx906_fa_amd_rope_cache_write_kv(
  * (5) Varlen direct-paged attention over the planar Q8 K+V cache: decode,
  *     chunked prefill, mixed batches and speculative verify in one call.
  *
- *     q    [num_tokens, Hq, D] (element strides), dtype fp16/bf16/fp32.
+ *     q    [num_tokens, Hq, D] (element strides), dtype fp16/bf16/fp32.  Rows
+ *          past the last sequence's are ignored (the decode kernels chosen for
+ *          a mixed batch are fewest where there are none).
  *     out  [num_tokens, Hq, D] (element strides), dtype fp32/fp16/bf16.
  *     Sequence s owns query tokens [query_start_loc[s], query_start_loc[s+1])
  *     and has seq_lens[s] cached tokens (the new ones included).
@@ -345,9 +347,9 @@ hipError_t gfx906_fa_amd_paged_attention_kv_write(
  *     padding tokens are written as zeros.  K bytes are permuted, never
  *     changed.  fp16 V sub-page layout: element (t, d) at byte
  *       2048*(d/64) + 32*(16*(t/4) + d%16) + 8*((d/16)%4) + 2*(t%4).
- *     Serves the contiguous entry gfx906_fa_forward
- *     (extension/gfx906_fa.cpp:120-265, launcher extension/gfx906_fa_launcher.cu:53-209),
- *     whose V stays fp16.
+ *     For callers that keep the repacked planes over several calls of (7);
+ *     gfx906_fa.forward (extension/gfx906_fa.cpp:120-265) makes one call of (9)
+ *     instead.
  */
 hipError_t gfx906_fa_amd_pack_flat_kv(const uint8_t *k_aos, const void *v_f16,
                                       uint8_t *k_planar, void *v_planar, int rows, int Skv,
@@ -382,7 +384,7 @@ hipError_t gfx906_fa_amd_paged_attention_tiled(
     int block_size, int max_query_len, float scale, float *out, int64_t out_token_stride,
     int64_t out_head_stride, hipStream_t stream);
 
-/* (7) Contiguous decode: the decode shapes of gfx906_fa_launch
+/* (8) Contiguous decode: the decode shapes of gfx906_fa_launch
  *     (extension/gfx906_fa_launcher.cu:53-209; gfx906_fa.forward with
  *     seq_q * num_heads / num_kv_heads <= 16 and no mask) on the reference's
  *     own contiguous layouts, with no repacking pass: k_q8 AoS Q8_0 rows
@@ -405,7 +407,7 @@ hipError_t gfx906_fa_amd_flat_decode(
     int num_kv_heads, int seq_kv, int head_size, float scale, float *out, int64_t out_token_stride,
     int64_t out_head_stride, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
-/* (8) Contiguous attention in one call (gfx906_fa_launch,
+/* (9) Contiguous attention in one call (gfx906_fa_launch,
  *     extension/gfx906_fa_launcher.cu:53-209; gfx906_fa.forward): q and out
  *     fp32 [batch][num_heads][seq_q][128], k_q8 AoS Q8_0 rows
  *     [batch][num_kv_heads][seq_kv][136 B], v_f16 fp16 rows
@@ -417,9 +419,16 @@ hipError_t gfx906_fa_amd_flat_decode(
  *     seq_q * num_heads / num_kv_heads <= 16) run as flat_decode, K and V
  *     16-byte aligned; others dequantize K and V once into tile images in the
  *     workspace (any alignment) and run the tiled kernel over them, long row
- *     tiles split over the keys.  workspace:
+ *     tiles split over the keys.  V rows of keys that no query row of a row
+ *     tile sees (past kv_max or its causal end) may then hold anything, Inf
+ *     and NaN included; decode shapes multiply all of kv_max rounded up to 16
+ *     keys, by 0 where unseen, so those V rows have to be finite.  workspace:
  *     gfx906_fa_amd_flat_attention_workspace_size() bytes, 256-byte aligned,
- *     no initial contents. */
+ *     no initial contents.  Past the decode shapes these are 35840 bytes of
+ *     images per 64 keys and kv-head (560 a key, of all seq_kv keys whatever
+ *     kv_max, with no cap; the planes of (6) take 392) and, where row tiles
+ *     may be split, their partials (up to 102 MB at 8 kv-heads): 59 MB for
+ *     2048 x 2048 at 8/4, 689 MB over 131072 keys at 64/8. */
 size_t gfx906_fa_amd_flat_attention_workspace_size(int batch, int seq_q, int num_heads, int num_kv_heads,
                                                    int seq_kv, int masked);
 hipError_t gfx906_fa_amd_flat_attention(
@@ -428,7 +437,7 @@ hipError_t gfx906_fa_amd_flat_attention(
     int num_heads, int num_kv_heads, int seq_kv, int head_size, float scale, float *out, void *workspace,
     size_t workspace_bytes, hipStream_t stream);
 
-/* (9) Padded-batch paged attention (gfx906_fa_launch_paged's own batch layout,
+/* (10) Padded-batch paged attention (gfx906_fa_launch_paged's own batch layout,
  *     extension/gfx906_fa.cpp:516-658): q [batch][num_heads][seq_q][128]
  *     (q_dtype) and out fp32 alike, both contiguous, over the planar cache as
  *     (5).  Without q_abs_offset every row sees all seq_lens[b] keys; with
@@ -436,7 +445,8 @@ hipError_t gfx906_fa_amd_flat_attention(
  *     with q_abs_offset; masked batches run the tiled kernel, split over the
  *     keys as (5)'s prefill is.  workspace:
  *     gfx906_fa_amd_paged_attention_padded_workspace_size() bytes, 256-byte
- *     aligned, no initial contents. */
+ *     aligned, no initial contents (a masked batch's: 102 MB of partials of
+ *     split row tiles, whatever its size; (7) takes masks without any). */
 size_t gfx906_fa_amd_paged_attention_padded_workspace_size(int batch, int seq_q, int num_heads, int num_kv_heads,
                                                            int max_seq_len, int masked);
 hipError_t gfx906_fa_amd_paged_attention_padded(

@@ -1,6 +1,7 @@
 """GPU: the contiguous entry ``gfx906_fa.forward`` (the reference's
 ``extension/gfx906_fa.cpp:120-265``: AoS Q8_0 K, fp16 V) against
-``oracle.flat_attention_ref``, and the repack kernels it uses, bit-exact."""
+``oracle.flat_attention_ref``, and the repack kernels of the C entry
+``gfx906_fa_amd_pack_flat_kv``, bit-exact."""
 import numpy as np
 import pytest
 import torch
